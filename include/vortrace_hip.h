@@ -13,9 +13,10 @@
  * RuntimeError).  vt_last_error() returns the message of the last failure on
  * the calling thread, with the reference's wording.
  *
- * A cloud owns per-cloud device work memory (the kernels' per-lane stacks,
- * the deferred-ray list, the adjoint's and field update's buffers, kept
- * between calls): calls on one cloud must not overlap in time; different
+ * A cloud owns per-cloud device memory: its tree, 260 bytes of neighbour lists
+ * per point, and work memory kept between calls (the kernels' per-lane stacks,
+ * the march's envelopes, at most 4.5 GiB, the deferred-ray list, the adjoint's
+ * and field update's buffers): calls on one cloud must not overlap in time; different
  * clouds may be used from different threads at once.
  *
  * Cell ids crossing the boundary are indices into the filtered particle list,
@@ -270,10 +271,13 @@ int vt_grid_rays(const vt_view *views, size_t nviews, double *d_start, double *d
 /* Launch parameters of the ray kernels (process-wide): lanes of a wave that
  * run their walk steps together, lanes that run their leaf steps together
  * (both 1..64), ray partitions (1, or 8: one per XCD), and help_events
- * (0..128): lanes with no ray left walk intervals of other lanes' rays of
- * their wave (sum, max, min and count kernels), recording up to this many
- * boundaries of one interval before they hand it back (0: off).  Results do
- * not depend on them, only speed.  No reference counterpart (the reference's
+ * (0..128).  With help_events > 0 rays are marched from cell to cell over the
+ * cells' neighbour lists, and the lanes of a wave share the check of the
+ * march -- 8 * help_events intervals at once, beyond which a ray is handed
+ * back -- and the ray engine, which runs the rays the march leaves, lets lanes
+ * with no ray left walk intervals of other lanes' rays, recording up to this
+ * many boundaries of one before they hand it back.  0: every ray runs in the
+ * engine, without help.  Results do not depend on them, only speed.  No reference counterpart (the reference's
  * OpenMP loop has schedule(dynamic,256) fixed, src/projection.cpp:43);
  * vortrace_amd.tuning.autotune picks them. */
 typedef struct {
@@ -293,9 +297,9 @@ int vt_cloud_lanes(const vt_cloud *cloud, int mode, int recorded, int64_t *lanes
 /* Per-call statistics of the last vt_project* call on this thread: total
  * segments (cell crossings), kNN queries run, the deepest walk and kNN
  * stacks, K_EXPAND searches, rays re-run by the K_EXPAND-capable kernel, the
- * kernels' time, and the intervals of rays walked by other lanes than the
- * ray's own (vt_tuning.help_events) and of those the ones handed back
- * unwalked. */
+ * kernels' time, and the intervals of rays walked or checked by other lanes
+ * than the ray's own (vt_tuning.help_events) and those handed back.  A march's
+ * queries are its start cells' and its searches of the tree. */
 typedef struct {
   int64_t segments, queries, max_walk_depth, max_knn_depth, slow_queries, deferred_rays;
   float kernel_ms;

@@ -70,6 +70,7 @@ struct Stats {
   unsigned long long part_counter[8];  // ray engine: work queue head per partition
   unsigned long long intervals;        // ray engine: intervals given to other lanes
   unsigned long long intervals_back;   // ... of which came back unwalked
+  unsigned long long fallback;         // march: rays left to the engine
 };
 
 // The ray engine splits its rays into kParts contiguous partitions, one per

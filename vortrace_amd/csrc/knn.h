@@ -43,7 +43,7 @@ constexpr int kLdsDepth = 16;
 // entries (68 dwords) starts the 16 lanes of a quarter-wave on 16 different
 // 4-bank groups, so 16-byte reads and writes at equal depth do not conflict.
 constexpr int kLdsStride = kLdsDepth + 1;
-__shared__ uint4 lds_stack[kBlock * kLdsStride];
+static __shared__ uint4 lds_stack[kBlock * kLdsStride];
 
 // A stack entry: tag, the lower bound `pb` of the box distances below it, and
 // a value (a box distance, or a saved dists[dim] for undo entries).

@@ -1,0 +1,1049 @@
+// The march's kernels: start cells, envelopes, and the replay of the
+// recursion that hands the segments on (march.h).
+#include <hip/hip_runtime.h>
+
+#include <algorithm>
+#include <cmath>
+#include <cstdint>
+
+#include "boxes.h"
+#include "engine.h"
+#include "march.h"
+#include "neighbors.h"
+
+#pragma clang fp contract(off)
+
+namespace vt {
+
+namespace {
+
+// What a third generator must stay clear of in r^2: the reference's tolerance
+// plus the rounding of squared distances between points of this size (the
+// expressions here and the reference's differ by some tens of roundings of
+// numbers up to scale^2).
+__device__ __forceinline__ double clearance(const DevCloud &C, const RayGeom &r, double &scale) {
+  double m = 0.0;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    m = fmax(m, fmax(fabs(r.a[d]), fabs(r.a[d] + r.len * r.d[d])));
+    m = fmax(m, fmax(fabs(C.rb_lo[d]), fabs(C.rb_hi[d])) + C.box[d]);
+  }
+  scale = m;
+  return 1.05 * kTol + 1e-14 * m * m;
+}
+
+__device__ __forceinline__ int64_t march_ray(const MarchRays &R, int64_t j) {
+  const int64_t k = R.base + j;
+  if (R.order) return (int64_t)gld(R.order + k);
+  return R.tile_row ? (int64_t)tile_ray((uint32_t)k, R.tile_row, R.tile_n) : k;
+}
+
+// 1 / b to about 1e-14.
+__device__ __forceinline__ double fast_rcp(double b) {
+  const double r = __builtin_amdgcn_rcp(b);
+  return __builtin_fma(r, __builtin_fma(-b, r, 1.0), r);
+}
+
+__device__ __forceinline__ uint32_t image_code(int x, int y, int z) {
+  return (uint32_t)((x + 1) * 9 + (y + 1) * 3 + (z + 1));
+}
+
+// Blocks are dealt to the XCDs in turn; give each XCD a contiguous share.
+__device__ __forceinline__ int64_t xcd_block(int64_t b, int64_t nb) {
+  const int64_t share = (nb + kParts - 1) / kParts;
+  return (b % kParts) * share + b / kParts;
+}
+
+// Every ray's start cell as entry 0 of its column, and 0 as the entry to march
+// from -- or kNone when the march cannot vouch for the start.  Also zeroes the
+// batch's queues.
+template <bool PER>
+__global__ __launch_bounds__(kBlock) void k_locate(DevCloud C, Scratch S, MarchRays R,
+                                                   MarchBufs B) {
+  const int tid = threadIdx.x;
+  const int gtid = blockIdx.x * kBlock + tid;
+  if (gtid < kMarchCounters) gst(B.ctr + gtid, 0u);
+  const LaneInfo li{tid, gtid, gtid >> 6, (int)(tid & 63)};
+  KStack st = make_stack(S, li);
+  for (int64_t j = gtid; j < R.n; j += (int64_t)gridDim.x * kBlock) {
+    const int64_t ray = march_ray(R, j);
+    RayGeom r;
+    make_ray(R.start + 3 * ray, R.end + 3 * ray, r);
+    uint32_t id[2];
+    double d[2];
+    query_reg<2, PER>(C, r.a[0], r.a[1], r.a[2], id, d, st);
+    double scale;
+    const double delta = clearance(C, r, scale);
+    const bool ok = id[0] != kNone && d[1] - d[0] > delta && r.len > 1e-6 && r.len < 1e30 &&
+                    !st.overflow;
+    if (ok) {
+      const uint32_t c0 = id[0];
+      uint32_t code = kNbCentre;
+      if constexpr (PER) {
+        // The generator's image nearest to the start.
+        const double2 xy = gld(reinterpret_cast<const double2 *>(C.gen + c0));
+        const double g[3] = {xy.x, xy.y, gld(&C.gen[c0].z)};
+        int im[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const double e = r.a[k] - g[k];
+          im[k] = e > 0.5 * C.box[k] ? 1 : (e < -0.5 * C.box[k] ? -1 : 0);
+        }
+        code = image_code(im[0], im[1], im[2]);
+      }
+      gst(B.seq + j, make_uint4(0u, 0u, c0 | (code << kNbSlotBits), 0u));
+    }
+    gst(B.c0 + j, ok ? 0u : kNone);
+  }
+}
+
+// A value from another lane of a group of 4 or 16: lanes 1 or 2 apart, or
+// mirrored within 8 or 16 (after the steps before, each of those lanes holds
+// its own quad's or half's result).
+template <int STEP>
+__device__ __forceinline__ uint32_t group_swap(uint32_t v) {
+  constexpr int ctrl = STEP == 0 ? 0xB1 : (STEP == 1 ? 0x4E : (STEP == 2 ? 0x141 : 0x140));
+  return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
+}
+template <int STEP>
+__device__ __forceinline__ double group_swap(double v) {
+  const uint64_t b = (uint64_t)__double_as_longlong(v);
+  const uint32_t lo = group_swap<STEP>((uint32_t)b), hi = group_swap<STEP>((uint32_t)(b >> 32));
+  return __longlong_as_double((long long)(((uint64_t)hi << 32) | lo));
+}
+
+// The nearest candidate (where it comes within the clearance, its g'.d and its
+// name) and the next one's place.
+struct Best {
+  double t1, h1, t2;
+  uint32_t n1;
+  __device__ __forceinline__ void clear() {
+    t1 = t2 = INFINITY;
+    h1 = 1.0;
+    n1 = kNone;
+  }
+  __device__ __forceinline__ void offer(double t, double h, uint32_t id, double next) {
+    const bool nearer = t < t1;
+    t2 = fmin(nearer ? t1 : t2, nearer ? next : t);
+    t1 = nearer ? t : t1;
+    h1 = nearer ? h : h1;
+    n1 = nearer ? id : n1;
+  }
+  template <int STEP>
+  __device__ __forceinline__ void swap_in() {
+    offer(group_swap<STEP>(t1), group_swap<STEP>(h1), group_swap<STEP>(n1), group_swap<STEP>(t2));
+  }
+  // The candidates of a group's lanes, in every lane.
+  template <int G>
+  __device__ __forceinline__ void reduce() {
+    swap_in<0>();
+    swap_in<1>();
+    if constexpr (G == 16) {
+      swap_in<2>();
+      swap_in<3>();
+    }
+  }
+};
+
+enum : int { kMpScan = 0, kMpBall = 1, kMpDone = 2 };
+
+// One ray's march.  Distances along the ray are relative to the entry of the
+// current cell c: with w = x(entry) - c, d the direction and g' = g - c, the
+// generator g becomes as near as c at tau = (|g'|^2 - 2 g'.w) / (2 g'.d), and
+// its squared distance less c's is 2 g'.d (tau_g - tau) there.  Candidates are
+// compared by where they come within the clearance, tau' (delta earlier in
+// r^2), so that the exit is verified when the next one's tau' lies beyond it.
+template <bool PER>
+struct Marcher {
+  RayGeom r;
+  double delta;
+  uint32_t c;    // current cell
+  double gb[3];  // its generator, in the primary box
+  int im[3];     // and image
+  double w[3];
+  double s, tend;  // entry of the cell, distance left on the ray
+  double tent;     // zone half-width at the entry
+  Best b;
+  int pos, k;
+
+  __device__ __forceinline__ void enter(const DevCloud &C, uint32_t cell, const double (&g)[3],
+                                        double at) {
+    c = cell;
+    s = at;
+    tend = r.len - at;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      gb[d] = g[d];
+      double p = g[d];
+      if (PER && im[d]) p = im[d] > 0 ? g[d] + C.box[d] : g[d] - C.box[d];
+      w[d] = (r.a[d] + at * r.d[d]) - p;
+    }
+    b.clear();
+    pos = 0;
+  }
+  // The exit (or infinity), relative to the entry.
+  __device__ __forceinline__ double exit_tau() const {
+    return b.n1 == kNone ? INFINITY : b.t1 + 0.5 * delta * fast_rcp(b.h1);
+  }
+  // Squared distance from c of the point tau after the entry.
+  __device__ __forceinline__ double r2_at(double tau) const {
+    double v2 = 0.0;
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      const double v = __builtin_fma(tau, r.d[d], w[d]);
+      v2 = __builtin_fma(v, v, v2);
+    }
+    return v2;
+  }
+  // tau' of a generator at e from c, and h = e.d; infinite when it recedes.
+  __device__ __forceinline__ double reach_of(const double (&e)[3], double &h, double &dd) const {
+    dd = __builtin_fma(e[2], e[2], __builtin_fma(e[1], e[1], e[0] * e[0]));
+    const double dw = __builtin_fma(e[2], w[2], __builtin_fma(e[1], w[1], e[0] * w[0]));
+    h = __builtin_fma(e[2], r.d[2], __builtin_fma(e[1], r.d[1], e[0] * r.d[0]));
+    const double t = (__builtin_fma(-2.0, dw, dd) - delta) * 0.5 * fast_rcp(h);
+    return h > 0.0 ? t : INFINITY;
+  }
+};
+
+// References of nodes still to be searched for an exit, per group, in LDS.
+constexpr int kBallStack = 128;
+
+// At most the squared distance from q to a box; q is the nearest float of a
+// point, which lies within `eps` of it along every axis.
+__device__ __forceinline__ float box_below2(const float (&lo)[3], const float (&hi)[3],
+                                            const float (&q)[3], float eps) {
+  float s = 0.0f;
+#pragma unroll
+  for (int d = 0; d < 3; ++d) {
+    const float t = fmaxf(fmaxf(lo[d] - q[d], q[d] - hi[d]) - eps, 0.0f);
+    s = __builtin_fmaf(t, t, s);
+  }
+  return s * 0.999999f;
+}
+
+// G lanes march one ray: each takes a share of every list chunk, and they hold
+// the ray's state alike.  4 lanes where rays are plentiful; 16 where they are
+// not, so that a crossing's chunk is read in one or two rounds.
+//
+// A cell whose list does not reach far enough for its exit has the tree
+// searched: boxes that touch the ball around the exit are opened, G at a time;
+// every generator found inside moves the exit closer and shrinks the ball (the
+// part of a ball ahead of the entry contains the later, smaller ones).  A
+// wave's rays wait until some need a search (or none can go on), so that the
+// searches' steps run for several rays at once.
+//
+// Groups take rays from a queue of the batch's slots, one part per XCD.
+//
+// Bound by FP64 issue: about 1,000 VALU instructions per 16 crossings.  2M
+// clustered cells, 512^2 rays (126 crossings each): 8.2 ms, of which the 1.4 %
+// of crossings that search take about half; a ray's own lane descending the
+// tree alone took 65 ms (chains of up to 300 dependent reads in clumps).
+template <bool PER, int G>
+__global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_march(DevCloud C, NbLists N, MarchRays R, MarchBufs B,
+                                              Stats *stats, int batch) {
+  constexpr int kShare = G == 4 ? 4 : 2;  // entries of a chunk per lane
+  constexpr int kChunk = G * kShare;
+  constexpr int kRays = 64 / G;
+  __shared__ uint32_t stack_all[kRays * kBallStack];
+  const int lane = threadIdx.x;
+  const int gl = lane & (G - 1), lead = lane & ~(G - 1);
+  uint32_t *stk = stack_all + (lane / G) * kBallStack;
+  const uint32_t below = (1u << gl) - 1u;
+  const uint64_t leads = G == 4 ? 0x1111111111111111ull : 0x0001000100010001ull;
+  auto slice = [&](uint64_t m) { return (uint32_t)(m >> lead) & ((1u << G) - 1u); };
+  Marcher<PER> M;
+  int ph = kMpDone;
+  int64_t j = 0;
+  double zone_c = 0.0;
+  uint32_t nball = 0;
+  // Ball search state (uniform in a group).
+  double bx[3] = {0.0, 0.0, 0.0}, br2 = 0.0, reach = 0.0;
+  uint32_t images = 0;
+  int code = 0, first = 0, sp = 0, steps = 0;
+  // The queue's parts, this block's own first.
+  const int64_t psize = (R.n + kParts - 1) / kParts;
+  int part = (int)(blockIdx.x & (kParts - 1));
+  int tries = 0;
+  bool more = true;  // the queue may hold rays (uniform in the wave)
+  for (;;) {
+    // Free groups take the next rays.
+    while (more) {
+      const uint64_t idle = __ballot(ph == kMpDone) & leads;
+      if (!idle) break;
+      const int need = __popcll(idle);
+      uint32_t base = 0;
+      if (lane == 0) base = atomicAdd(B.ctr + part, (uint32_t)need);
+      base = __shfl(base, 0);
+      const int64_t lo = part * psize, hi = min(lo + psize, R.n);
+      const int64_t at = lo + base + __popcll(idle & ((1ull << lead) - 1ull));
+      if (ph == kMpDone && ((idle >> lead) & 1ull) && at < hi) {
+        j = at;
+        const uint32_t k = gld(B.c0 + j);
+        if (k == kNone) {
+          if (gl == 0) gst(B.c0 + j, 0u);
+        } else {
+          const int64_t ray = march_ray(R, j);
+          make_ray(R.start + 3 * ray, R.end + 3 * ray, M.r);
+          double scale;
+          M.delta = clearance(C, M.r, scale);
+          zone_c = 1e-13 * scale;
+          const uint4 e = gld(B.seq + (size_t)k * B.stride + j);
+          const uint32_t slot = e.z & kNbSlotMask;
+          const int ic = (int)(e.z >> kNbSlotBits);
+          const double2 xy = gld(reinterpret_cast<const double2 *>(C.gen + slot));
+          const double g[3] = {xy.x, xy.y, gld(&C.gen[slot].z)};
+          M.im[0] = ic / 9 - 1;
+          M.im[1] = (ic / 3) % 3 - 1;
+          M.im[2] = ic % 3 - 1;
+          M.k = (int)k;
+          M.tent = (double)__uint_as_float(e.w);
+          M.enter(C, slot, g,
+                  __longlong_as_double((long long)(((uint64_t)e.y << 32) | e.x)));
+          ph = kMpScan;
+        }
+      }
+      if (lo + base + need >= hi) {
+        // This part is used up.
+        part = (part + 1) & (kParts - 1);
+        more = ++tries < kParts;
+      }
+    }
+    const uint64_t scan = __ballot(ph == kMpScan), wait = __ballot(ph == kMpBall);
+    if (!(scan | wait)) break;
+    bool settle = false;  // the exit is certain: cross (or end)
+    const bool search = __popcll(wait) >= batch * G || !scan;
+    if (ph == kMpScan && !search) {
+      // One chunk of the cell's list, this lane's share of it.
+      const uint32_t *list = N.nb + (size_t)M.c * kNbMax + kChunk * M.pos + kShare * gl;
+      uint32_t id[kShare];
+      if constexpr (kShare == 4) {
+        const uint4 q = gld(reinterpret_cast<const uint4 *>(list));
+        id[0] = q.x;
+        id[1] = q.y;
+        id[2] = q.z;
+        id[3] = q.w;
+      } else {
+        const uint64_t q = gld(reinterpret_cast<const uint64_t *>(list));
+        id[0] = (uint32_t)q;
+        id[1] = (uint32_t)(q >> 32);
+      }
+      double2 gxy[kShare];
+      double gz[kShare];
+#pragma unroll
+      for (int i = 0; i < kShare; ++i) {
+        const uint32_t sl = id[i] == kNone ? M.c : (id[i] & kNbSlotMask);
+        gxy[i] = gld(reinterpret_cast<const double2 *>(C.gen + sl));
+        gz[i] = gld(&C.gen[sl].z);
+      }
+      double last = 0.0;
+      Best b;
+      b.clear();
+#pragma unroll
+      for (int i = 0; i < kShare; ++i) {
+        double e[3] = {gxy[i].x - M.gb[0], gxy[i].y - M.gb[1], gz[i] - M.gb[2]};
+        bool valid = id[i] != kNone;
+        if constexpr (PER) {
+          const uint32_t rc = id[i] >> kNbSlotBits;
+          if (valid && rc != kNbCentre) {
+            const int sh[3] = {(int)(rc / 9) - 1, (int)(rc / 3) % 3 - 1, (int)(rc % 3) - 1};
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+              e[d] += sh[d] * C.box[d];
+              valid &= abs(M.im[d] + sh[d]) <= 1;
+            }
+          }
+        }
+        double h, dd;
+        const double t = M.reach_of(e, h, dd);
+        b.offer(valid ? t : INFINITY, h, id[i], INFINITY);
+        last = id[i] == kNone ? INFINITY : dd;
+      }
+      b.template reduce<G>();
+      M.b.offer(b.t1, b.h1, b.n1, b.t2);
+      last = __shfl(last, lead + G - 1);  // the chunk's farthest
+      ++M.pos;
+      // Generators not seen yet are at least `lim` from c.
+      const bool ended = last == INFINITY || M.pos == kNbMax / kChunk;
+      const double lim = ended ? (double)gld(N.r2 + M.c) : last * 0.999998;
+      const double v2 = M.r2_at(fmin(M.exit_tau(), M.tend));
+      // Empty ball: |x - g| >= |g - c| - |x - c|, so none of them is within
+      // the clearance of the exit when D^2 - delta > 2 D |x - c|.
+      const double q = lim - M.delta;
+      if (q > 0.0 && q * q > 4.000008 * lim * v2) {
+        settle = true;
+      } else if (ended) {
+        ph = kMpBall;
+        reach = 2.0 * sqrt(lim);
+        images = 0;
+        sp = -1;  // the search has not begun
+        steps = 0;
+      }
+    }
+    // The waiting rays' searches, until all of them have ended.
+    while (search && __ballot(ph == kMpBall && !settle)) {
+      const bool on = ph == kMpBall && !settle;
+      auto centre = [&]() {
+        // The ball around the exit known so far, no farther than `reach` while
+        // there is none.
+        const double te = M.exit_tau();
+        const double tx = fmin(M.b.n1 == kNone ? reach : te, M.tend);
+        br2 = M.delta;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const double v = __builtin_fma(tx, M.r.d[d], M.w[d]);
+          br2 = __builtin_fma(v, v, br2);
+          double p = M.gb[d];
+          if (PER && M.im[d]) p += M.im[d] * C.box[d];
+          bx[d] = p + v;
+        }
+      };
+      auto shift = [&](int d) {
+        return (double)(d == 0 ? code / 9 - 1 : (d == 1 ? (code / 3) % 3 - 1 : code % 3 - 1)) *
+               C.box[d];
+      };
+      if (on && sp < 0) {
+        if (gl == 0) ++nball;
+        centre();
+        sp = 0;
+        images = 1u << kNbCentre;
+        first = (int)kNbCentre;
+        if constexpr (PER) {
+          // Images whose generators can be within the ball, the nearest first.
+          uint32_t ms[3];
+          const double r = sqrt(br2);
+          first = 0;
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            ms[d] = 0u;
+            double nearest = DBL_MAX;
+            int at = 1;
+#pragma unroll
+            for (int k = -1; k <= 1; ++k) {
+              const double q = bx[d] - k * C.box[d];
+              const double o = fmax(fmax(C.rb_lo[d] - q, q - C.rb_hi[d]), 0.0);
+              if (o <= r) ms[d] |= 1u << (k + 1);
+              if (o < nearest) {
+                nearest = o;
+                at = k + 1;
+              }
+            }
+            first = 3 * first + at;
+          }
+          images = 0u;
+#pragma unroll
+          for (int a = 0; a < 3; ++a)
+#pragma unroll
+            for (int b = 0; b < 3; ++b)
+              if (((ms[0] >> a) & (ms[1] >> b) & 1u) != 0u) images |= ms[2] << (a * 9 + b * 3);
+        }
+      }
+      if (on && sp == 0 && images) {
+        // The next image: its root.
+        code = first;
+        if (!((images >> code) & 1u)) code = __ffs(images) - 1;
+        images &= ~(1u << code);
+        if (gl == 0) stk[0] = C.root;
+        sp = 1;
+      }
+      __builtin_amdgcn_wave_barrier();
+      __threadfence_block();
+      // The centre in the image's frame, and what its floats may be off.
+      double q1[3];
+      float qf[3], eps = 0.0f;
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        q1[d] = PER ? bx[d] - shift(d) : bx[d];
+        qf[d] = (float)q1[d];
+        eps = fmaxf(eps, fabsf(qf[d]) * 1.2e-7f);
+      }
+      const float bf = (float)br2 * 1.000001f;
+      const int take = on ? min(sp, G) : 0;
+      uint32_t ref = 0u;
+      const bool have = gl < take;
+      if (have) ref = stk[sp - take + gl];
+      sp -= take;
+      const bool leaf = have && (ref & kRefLeaf);
+      const bool inner = have && !(ref & kRefLeaf);
+      uint32_t kn = 0u, kf = 0u;
+      bool pn = false, pf = false;
+      if (inner) {
+        const uint4 *p = reinterpret_cast<const uint4 *>(N.boxes + ref);
+        const uint4 v0 = gld(p), v1 = gld(p + 1), v2 = gld(p + 2), v3 = gld(p + 3);
+        const float lo1[3] = {__uint_as_float(v0.x), __uint_as_float(v0.y), __uint_as_float(v0.z)};
+        const float hi1[3] = {__uint_as_float(v0.w), __uint_as_float(v1.x), __uint_as_float(v1.y)};
+        const float lo2[3] = {__uint_as_float(v1.z), __uint_as_float(v1.w), __uint_as_float(v2.x)};
+        const float hi2[3] = {__uint_as_float(v2.y), __uint_as_float(v2.z), __uint_as_float(v2.w)};
+        const float d1 = box_below2(lo1, hi1, qf, eps), d2 = box_below2(lo2, hi2, qf, eps);
+        const bool first1 = d1 <= d2;
+        kn = first1 ? v3.x : v3.y;
+        kf = first1 ? v3.y : v3.x;
+        pn = fminf(d1, d2) < bf;
+        pf = fmaxf(d1, d2) < bf;
+      }
+      // Far children below near ones: the near ones are taken next.
+      const uint32_t mf = slice(__ballot(pf)), mn = slice(__ballot(pn));
+      const int nf = __popc(mf), nn = __popc(mn);
+      bool fail = on && (sp + nf + nn > kBallStack || ++steps > 8192);
+      if (!fail) {
+        if (pf) stk[sp + __popc(mf & below)] = kf;
+        if (pn) stk[sp + nf + __popc(mn & below)] = kn;
+        sp += nf + nn;
+      }
+      bool found = false;
+      Best b;
+      b.clear();
+      if (leaf) {
+        const uint32_t s0 = ref & kSlotMask;
+        const uint32_t end = (uint32_t)gld(&C.gen[s0].end);
+        // The current candidate under its absolute name.
+        uint32_t nslot = kNone;
+        int ncode = (int)kNbCentre;
+        if (M.b.n1 != kNone) {
+          nslot = M.b.n1 & kNbSlotMask;
+          if constexpr (PER) {
+            const int rc = (int)(M.b.n1 >> kNbSlotBits);
+            ncode = (M.im[0] + rc / 9) * 9 + (M.im[1] + (rc / 3) % 3) * 3 + M.im[2] + rc % 3;
+          }
+        }
+        const int ccode = PER ? (int)image_code(M.im[0], M.im[1], M.im[2]) : (int)kNbCentre;
+        // Half a leaf at a time, its loads in flight together (past the
+        // leaf's end they stay within the padding records).
+#pragma unroll
+        for (int h0 = 0; h0 < kLeafMaxSize; h0 += kLeafChunk) {
+          if (h0 && s0 + h0 >= end) break;
+          double2 xy[kLeafChunk];
+          double z[kLeafChunk];
+#pragma unroll
+          for (int i = 0; i < kLeafChunk; ++i) {
+            xy[i] = gld(reinterpret_cast<const double2 *>(C.gen + s0 + h0 + i));
+            z[i] = gld(&C.gen[s0 + h0 + i].z);
+          }
+          uint32_t in = 0u;
+#pragma unroll
+          for (int i = 0; i < kLeafChunk; ++i) {
+            const uint32_t t = s0 + (uint32_t)(h0 + i);
+            const double e0 = q1[0] - xy[i].x, e1 = q1[1] - xy[i].y, e2 = q1[2] - z[i];
+            const double d2 = __builtin_fma(e2, e2, __builtin_fma(e1, e1, e0 * e0));
+            if (t < end && d2 < br2 && !(t == M.c && code == ccode) &&
+                !(t == nslot && code == ncode))
+              in |= 1u << i;
+          }
+          while (in) {
+            const uint32_t t = s0 + (uint32_t)(h0 + __ffs(in) - 1);
+            in &= in - 1u;
+            const double2 gxy = gld(reinterpret_cast<const double2 *>(C.gen + t));
+            double g[3] = {gxy.x - M.gb[0], gxy.y - M.gb[1], gld(&C.gen[t].z) - M.gb[2]};
+            int rel[3] = {0, 0, 0};
+            if constexpr (PER) {
+              rel[0] = code / 9 - 1 - M.im[0];
+              rel[1] = (code / 3) % 3 - 1 - M.im[1];
+              rel[2] = code % 3 - 1 - M.im[2];
+#pragma unroll
+              for (int d = 0; d < 3; ++d) g[d] += rel[d] * C.box[d];
+            }
+            double h, dd;
+            const double tv = M.reach_of(g, h, dd);
+            // A generator that recedes, or two images away, is no exit the
+            // march can name: leave the ray to the engine.
+            if (tv == INFINITY || abs(rel[0]) > 1 || abs(rel[1]) > 1 || abs(rel[2]) > 1)
+              fail = true;
+            else
+              b.offer(tv, h, t | (image_code(rel[0], rel[1], rel[2]) << kNbSlotBits), INFINITY);
+            found = true;
+          }
+        }
+      }
+      if (slice(__ballot(fail))) {
+        if (gl == 0) gst(B.c0 + j, 0u);
+        ph = kMpDone;
+      } else if (slice(__ballot(found))) {
+        b.template reduce<G>();
+        M.b.offer(b.t1, b.h1, b.n1, b.t2);
+        centre();
+      }
+      if (ph == kMpBall && sp == 0 && !images) {
+        if (M.b.n1 == kNone && reach < M.tend) {
+          reach *= 4.0;
+          sp = -1;
+        } else {
+          settle = true;
+        }
+      }
+    }
+    if (settle) {
+      const double te = M.exit_tau();
+      int cells = 0;  // 0: left to the engine
+      bool done = true;
+      // Each boundary's generators must be the images nearest to every point
+      // of the two cells' chords.
+      double lim = DBL_MAX;
+      if constexpr (PER) {
+        lim = 0.2 * fmin(C.box[0], fmin(C.box[1], C.box[2]));
+        lim = M.r2_at(0.0) < lim * lim ? lim : 0.0;
+      }
+      if (!(M.b.t1 <= M.tend)) {
+        // The ray ends in this cell, clear of its entry.
+        if (M.tend > M.tent && M.tend < lim && M.r2_at(M.tend) < lim * lim) cells = M.k + 1;
+      } else {
+        const uint32_t n = M.b.n1 & kNbSlotMask;
+        const int rc = (int)(M.b.n1 >> kNbSlotBits);
+        const double2 xy = gld(reinterpret_cast<const double2 *>(C.gen + n));
+        const double g[3] = {xy.x, xy.y, gld(&C.gen[n].z)};
+        double p1[3], p2[3];
+        const int sh[3] = {rc / 9 - 1, (rc / 3) % 3 - 1, rc % 3 - 1};
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          p1[d] = M.gb[d];
+          p2[d] = g[d];
+          if constexpr (PER) {
+            if (M.im[d]) p1[d] = M.im[d] > 0 ? M.gb[d] + C.box[d] : M.gb[d] - C.box[d];
+            const int i2 = M.im[d] + sh[d];
+            if (i2) p2[d] = i2 > 0 ? g[d] + C.box[d] : g[d] - C.box[d];
+          }
+        }
+        const double sv = split_analytic(M.r, p1, p2);
+        const double zone = 0.5 * M.delta * fast_rcp(M.b.h1) * 1.000001 + zone_c;
+        const double chord = sv - M.s;
+        const bool ok = te < M.b.t2 && te < M.tend && M.b.h1 > 1e-10 && fabs(chord - te) <= zone &&
+                        chord > M.tent + zone && chord < lim && M.r2_at(te) < lim * lim &&
+                        n != M.c && M.k + 1 < B.cap;
+        if (ok) {
+          ++M.k;
+          // The next float up keeps the stored half-width at least the zone.
+          const float zf = __uint_as_float(__float_as_uint((float)zone) + 1u);
+          M.tent = (double)zf;
+          if constexpr (PER) {
+#pragma unroll
+            for (int d = 0; d < 3; ++d) M.im[d] += sh[d];
+          }
+          const uint32_t ic = PER ? image_code(M.im[0], M.im[1], M.im[2]) : kNbCentre;
+          const uint64_t sb = (uint64_t)__double_as_longlong(sv);
+          if (gl == 0)
+            gst(B.seq + (size_t)M.k * B.stride + j,
+                make_uint4((uint32_t)sb, (uint32_t)(sb >> 32), n | (ic << kNbSlotBits),
+                           __float_as_uint(zf)));
+          M.enter(C, n, g, sv);
+          ph = kMpScan;
+          done = false;
+        }
+      }
+      if (done) {
+        if (gl == 0) gst(B.c0 + j, (uint32_t)cells);
+        ph = kMpDone;
+      }
+    }
+  }
+  for (int o = 32; o; o >>= 1) nball += __shfl_xor(nball, o);
+  if (lane == 0 && nball) atomicAdd(&stats->queries, (unsigned long long)nball);
+}
+
+// A ray's records start at the place its wave reserved for it.
+template <class IO>
+struct Finish {
+  using Sink = typename IO::Sink;
+  static __device__ __forceinline__ void reserve(const IO &, Sink &, int, int) {}
+  static __device__ __forceinline__ void begin(const IO &io, int64_t ray, Sink &sk) {
+    io.begin(ray, sk);
+  }
+  static __device__ __forceinline__ int end(const IO &io, int64_t ray, Sink &sk) {
+    return io.end(ray, sk);
+  }
+};
+template <class Inner>
+struct MarchRecSink : Inner::Sink {
+  RecPool pool;
+  unsigned long long next;
+  uint32_t ray;
+  __device__ __forceinline__ void seg(uint32_t cell, double a, double b) {
+    const uint32_t k = (uint32_t)this->n;
+    Inner::Sink::seg(cell, a, b);
+    if (next < pool.cap) {
+      SegRec *q = pool.rec + next;
+      gst_nt(reinterpret_cast<uint4 *>(q), make_uint4(cell, ray, k, 0u));
+      gst_nt(&q->ds, b - a);
+    } else {
+      atomicOr(pool.overflow, 1);
+    }
+    ++next;
+  }
+};
+template <class Inner>
+struct Finish<MarchRecordIO<Inner>> {
+  using IO = MarchRecordIO<Inner>;
+  using Sink = MarchRecSink<Inner>;
+  // The wave takes one run of whole chunks, its rays' records in lane order;
+  // the last lanes mark the rest of the last chunk unwritten.
+  static __device__ __forceinline__ void reserve(const IO &io, Sink &sk, int cells, int lane) {
+    int inc = cells;
+    for (int o = 1; o < 64; o <<= 1) {
+      const int v = __shfl_up(inc, o);
+      if (lane >= o) inc += v;
+    }
+    const int total = __shfl(inc, 63);
+    const int whole = (total + kRecChunk - 1) / kRecChunk * kRecChunk;
+    unsigned long long base = 0;
+    if (lane == 0 && whole) base = atomicAdd(io.pool.head, (unsigned long long)whole);
+    base = __shfl(base, 0);
+    sk.pool = io.pool;
+    sk.next = base + (unsigned long long)(inc - cells);
+    const unsigned long long rest = base + (unsigned long long)total + (unsigned long long)lane;
+    if (lane < whole - total && rest < io.pool.cap) gst(&io.pool.rec[rest].ray, kNone);
+  }
+  static __device__ __forceinline__ void begin(const IO &io, int64_t ray, Sink &sk) {
+    io.inner.begin(ray, static_cast<typename Inner::Sink &>(sk));
+    sk.ray = (uint32_t)ray;
+  }
+  static __device__ __forceinline__ int end(const IO &io, int64_t ray, Sink &sk) {
+    return io.inner.end(ray, static_cast<typename Inner::Sink &>(sk));
+  }
+};
+
+// Intervals a wave can hold for its lanes (64-bit items in LDS).
+constexpr int kPool = 1024;
+
+// The replay of the recursion (see march.h) over the lanes of a wave, then the
+// segments.  An item is an interval (i, j), j >= i + 2, of a ray's cells that
+// the recursion visits as a pair; its split point inserts a cell k between
+// them and leaves (i, k) and (k, j).  Intervals do not depend on one another,
+// so any lane takes any interval of the wave's rays: lanes without a ray, or
+// whose ray is done, work on the others'.  Bound by the latency of the entries'
+// reads, one column per ray (2.7 ms at 512^2 rays, 2M clustered cells).
+template <bool PER, class IO>
+__global__ __launch_bounds__(64) void k_finish(DevCloud C, MarchRays R, MarchBufs B, int rpw,
+                                               int pool, IO io, uint32_t *fall, ErrRec *err,
+                                               Stats *stats) {
+  __shared__ uint64_t item[kPool];
+  __shared__ double geo[7][64];
+  __shared__ int cells[64];
+  __shared__ uint32_t bad[64];
+  const int lane = threadIdx.x;
+  const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
+  const int64_t j0 = blk * rpw;
+  const int64_t j = j0 + lane;
+  const bool mine = lane < rpw && j < R.n;
+  int K = 0;
+  int64_t ray = 0;
+  RayGeom r;
+  uint64_t first[2] = {0, 0};
+  int nfirst = 0;
+  if (mine) {
+    ray = march_ray(R, j);
+    K = (int)gld(B.c0 + j);
+    make_ray(R.start + 3 * ray, R.end + 3 * ray, r);
+#pragma unroll
+    for (int d = 0; d < 3; ++d) {
+      geo[d][lane] = r.a[d];
+      geo[3 + d][lane] = r.d[d];
+    }
+    geo[6][lane] = r.len;
+  }
+  bool fail = mine && K == 0;
+  auto entry = [&](int64_t col, int k) { return gld(B.seq + (size_t)k * B.stride + col); };
+  auto at = [](const uint4 &e) {
+    return __longlong_as_double((long long)(((uint64_t)e.y << 32) | e.x));
+  };
+  // The cell k of [lo, hi] that s falls in, clear of both its boundaries.
+  auto locate = [&](int64_t col, int n, double len, double s, int lo, int hi, uint4 &ek) {
+    ek = entry(col, lo);
+    if (s < at(ek)) return -1;
+    while (hi > lo) {
+      const int mid = (lo + hi + 1) >> 1;
+      const uint4 em = entry(col, mid);
+      if (at(em) <= s) {
+        lo = mid;
+        ek = em;
+      } else {
+        hi = mid - 1;
+      }
+    }
+    double next = len, zn = 0.0;
+    if (lo + 1 < n) {
+      const uint4 en = entry(col, lo + 1);
+      next = at(en);
+      zn = (double)__uint_as_float(en.w);
+    }
+    const double zk = lo > 0 ? (double)__uint_as_float(ek.w) : -1.0;
+    return (s - at(ek) > zk && next - s > zn) ? lo : -1;
+  };
+  auto pack = [](int owner, int depth, int i, int k) {
+    return (uint64_t)owner | ((uint64_t)depth << 8) | ((uint64_t)i << 16) | ((uint64_t)k << 32);
+  };
+  if (mine && K > 0) {
+    const uint32_t a = entry(j, 0).z & kNbSlotMask, b = entry(j, K - 1).z & kNbSlotMask;
+    if constexpr (PER) {
+      gst(B.ins + j, 0.0);
+      gst(B.ins + (size_t)(K - 1) * B.stride + j, r.len);
+      if (a == b) {
+        // Same cell at both ends: dyadic probes for another one
+        // (src/ray.cpp:220-246).
+        fail = true;
+        bool go = K > 1;
+        for (int lv = 1; go && lv <= 10; ++lv)
+          for (int i = 1; go && i < (1 << lv); i += 2) {
+            const double mid = r.len * i / (1 << lv);
+            uint4 ek;
+            const int k = locate(j, K, r.len, mid, 0, K - 1, ek);
+            if (k < 0) {
+              go = false;
+            } else if ((ek.z & kNbSlotMask) != a) {
+              go = false;
+              fail = false;
+              gst(B.ins + (size_t)k * B.stride + j, mid);
+              if (k >= 2) first[nfirst++] = pack(lane, 1, 0, k);
+              if (K - 1 - k >= 2) first[nfirst++] = pack(lane, 0, k, K - 1);
+            }
+          }
+      } else if (K >= 3) {
+        first[nfirst++] = pack(lane, 0, 0, K - 1);
+      }
+    } else {
+      fail = a == b && K > 1;
+      if (!fail && K >= 3) first[nfirst++] = pack(lane, 0, 0, K - 1);
+    }
+  }
+  cells[lane] = K;
+  bad[lane] = 0u;
+  __syncthreads();
+  int count = 0;
+  uint32_t given = 0, back = 0;
+#pragma unroll
+  for (int q = 0; q < 2; ++q) {
+    const bool put = nfirst > q;
+    const uint64_t m = __ballot(put);
+    const int p = count + __popcll(m & ((1ull << lane) - 1ull));
+    if (put) {
+      if (p < pool) {
+        item[p] = first[q];
+      } else {
+        bad[lane] = 1u;
+        ++back;
+      }
+    }
+    count = min(pool, count + (int)__popcll(m));
+  }
+  __syncthreads();
+  while (count > 0) {
+    const int take = count < 64 ? count : 64;
+    count -= take;
+    uint64_t it = 0;
+    const bool work = lane < take;
+    if (work) it = item[count + lane];
+    __syncthreads();
+    uint64_t child[2] = {0, 0};
+    bool put[2] = {false, false};
+    int owner = 0;
+    if (work) {
+      owner = (int)(it & 255u);
+      const int depth = (int)((it >> 8) & 255u);
+      const int i = (int)((it >> 16) & 0xFFFFu), jj = (int)((it >> 32) & 0xFFFFu);
+      if (owner != lane) ++given;
+      if (!bad[owner]) {
+        const int64_t col = j0 + owner;
+        const int n = cells[owner];
+        RayGeom g;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          g.a[d] = geo[d][owner];
+          g.d[d] = geo[3 + d][owner];
+        }
+        g.len = geo[6][owner];
+        const uint32_t ci = entry(col, i).z & kNbSlotMask, cj = entry(col, jj).z & kNbSlotMask;
+        bool ok = ci != cj && depth < 120;
+        double s = 0.0, p1[3], p2[3];
+        double sc = 0.0, sn = g.len;
+        if constexpr (PER) {
+          sc = gld(B.ins + (size_t)i * B.stride + col);
+          sn = gld(B.ins + (size_t)jj * B.stride + col);
+        }
+        bool analytic = split_point<PER>(C, g, ci, cj, sc, sn, s, p1, p2);
+        int k = -1;
+        uint4 ek;
+        if (ok && analytic) {
+          if constexpr (PER) {
+            const double l2 = sc + 1e-15, h2 = sn - 1e-15;
+            s = (s < l2) ? l2 : ((h2 < s) ? h2 : s);
+          }
+          k = locate(col, n, g.len, s, i, jj, ek);
+        } else if (PER && ok) {
+          // The reference's bisection between the two cells.
+          double lo = sc, hi = sn;
+          for (int q = 0; q < 64; ++q) {
+            const double mid = 0.5 * (lo + hi);
+            const int km = locate(col, n, g.len, mid, i, jj, ek);
+            if (km < 0) break;
+            const uint32_t cm = ek.z & kNbSlotMask;
+            if (cm != ci && cm != cj) {
+              const double l2 = sc + 1e-15, h2 = sn - 1e-15;
+              s = (mid < l2) ? l2 : ((h2 < mid) ? h2 : mid);
+              k = s == mid ? km : -1;
+              break;
+            }
+            if (cm == ci)
+              lo = mid;
+            else
+              hi = mid;
+            if (hi - lo < 1e-11) break;
+          }
+        }
+        if (k <= i || k >= jj) {
+          ok = false;
+        } else {
+          const uint32_t ck = ek.z & kNbSlotMask;
+          ok = ok && ck != ci && ck != cj;
+        }
+        if (!ok) {
+          bad[owner] = 1u;
+        } else {
+          if constexpr (PER) gst(B.ins + (size_t)k * B.stride + col, s);
+          put[0] = jj - k >= 2;
+          child[0] = pack(owner, depth, k, jj);
+          put[1] = k - i >= 2;
+          child[1] = pack(owner, depth + 1, i, k);
+        }
+      }
+    }
+    // Insertion points written here are read by whichever lane takes the
+    // children.
+    __threadfence_block();
+#pragma unroll
+    for (int q = 0; q < 2; ++q) {
+      const uint64_t m = __ballot(put[q]);
+      const int p = count + __popcll(m & ((1ull << lane) - 1ull));
+      if (put[q]) {
+        if (p < pool) {
+          item[p] = child[q];
+        } else {
+          bad[owner] = 1u;  // no room: the engine walks the ray
+          ++back;
+        }
+      }
+      count = min(pool, count + (int)__popcll(m));
+    }
+    __syncthreads();
+  }
+  fail |= mine && bad[lane] != 0u;
+  const int out = mine && !fail ? K : 0;
+  using F = Finish<IO>;
+  typename F::Sink sk;
+  F::reserve(io, sk, out, lane);
+  if (out > 0) {
+    F::begin(io, ray, sk);
+    uint4 e = entry(j, 0);
+    for (int k = 0; k < out; ++k) {
+      uint4 nx = e;
+      double b = r.len;
+      if (k + 1 < out) {
+        nx = entry(j, k + 1);
+        b = at(nx);
+      }
+      sk.seg(e.z & kNbSlotMask, at(e), b);
+      e = nx;
+    }
+    const int rc = F::end(io, ray, sk);
+    if (rc) report_error(err, rc, ray, 0.0, 0.0, 0.0, 0u, 0u);
+  } else if (fail) {
+    const unsigned long long q = atomicAdd(&stats->fallback, 1ull);
+    gst(fall + q, (uint32_t)ray);
+  }
+  uint64_t seg = (uint64_t)out;
+  for (int o = 32; o; o >>= 1) {
+    seg += __shfl_xor(seg, o);
+    given += __shfl_xor(given, o);
+    back += __shfl_xor(back, o);
+  }
+  if (lane == 0) {
+    atomicAdd(&stats->segments, (unsigned long long)seg);
+    if (given) atomicAdd(&stats->intervals, (unsigned long long)given);
+    if (back) atomicAdd(&stats->intervals_back, (unsigned long long)back);
+  }
+}
+
+}  // namespace
+
+// Rays a wave marches: all its lanes' when there are rays for every SIMD, else
+// fewer, so that the rays spread over the chip.
+int march_rays_per_wave(int64_t n, int cus) {
+  int rpw = 64;
+  while (rpw > 4 && (n + rpw - 1) / rpw < 8ll * cus) rpw >>= 1;
+  return rpw;
+}
+
+// Waves of a batch: a multiple of kParts, so that every XCD has the same share.
+int64_t march_waves(int64_t n, int cus) {
+  const int rpw = march_rays_per_wave(n, cus);
+  return ((n + rpw - 1) / rpw + kParts - 1) / kParts * kParts;
+}
+
+void march_build_lists(const DevCloud &C, uint32_t *nb, float *r2, hipStream_t st) {
+  const unsigned grid = (C.n + kNbWindow - 1) / kNbWindow;
+  if (C.periodic)
+    k_neighbors<true><<<grid, 64, 0, st>>>(C, nb, r2);
+  else
+    k_neighbors<false><<<grid, 64, 0, st>>>(C, nb, r2);
+}
+
+void march_build_boxes(const DevCloud &C, uint32_t nodes, BNode *boxes, uint32_t *work,
+                       hipStream_t st) {
+  if (!nodes) return;
+  uint32_t *parent = work, *arrived = work + nodes, *leaf_parent = work + 2 * (size_t)nodes;
+  k_box_parents<<<(nodes + 255) / 256, 256, 0, st>>>(C.nodes, nodes, C.root, boxes, parent,
+                                                     leaf_parent, arrived);
+  k_box_climb<<<(C.n + 255) / 256, 256, 0, st>>>(C.gen, C.n, boxes, parent, leaf_parent, arrived);
+}
+
+int march_locate_grid(int cus) { return 4 * cus; }
+
+template <bool PER>
+static void march_batch_p(const MarchCall &m) {
+  const int grid = (int)std::min<int64_t>(march_locate_grid(m.cus), (m.R.n + kBlock - 1) / kBlock);
+  k_locate<PER><<<grid, kBlock, 0, m.st>>>(m.C, m.S, m.R, m.B);
+  // As many waves as the chip holds at once, or as the rays need.
+  if (m.R.n >= 64ll * m.cus) {
+    const unsigned waves = (unsigned)std::min<int64_t>(16ll * m.cus, (m.R.n + 15) / 16);
+    k_march<PER, 4><<<waves, 64, 0, m.st>>>(m.C, m.N, m.R, m.B, m.stats, 4);
+  } else {
+    k_march<PER, 16><<<(unsigned)((m.R.n + 3) / 4), 64, 0, m.st>>>(m.C, m.N, m.R, m.B, m.stats, 1);
+  }
+}
+
+void march_batch(const MarchCall &m, bool periodic) {
+  if (periodic)
+    march_batch_p<true>(m);
+  else
+    march_batch_p<false>(m);
+}
+
+template <class IO>
+void march_finish(const MarchCall &m, bool periodic, const IO &io) {
+  const int rpw = march_rays_per_wave(m.R.n, m.cus);
+  const int64_t nb = march_waves(m.R.n, m.cus);
+  const int pool = std::min(m.pool, kPool);
+  if (periodic)
+    k_finish<true, IO><<<(unsigned)nb, 64, 0, m.st>>>(m.C, m.R, m.B, rpw, pool, io, m.fall, m.err,
+                                                      m.stats);
+  else
+    k_finish<false, IO><<<(unsigned)nb, 64, 0, m.st>>>(m.C, m.R, m.B, rpw, pool, io, m.fall, m.err,
+                                                       m.stats);
+}
+
+#define VT_FINISH(...) template void march_finish<__VA_ARGS__>(const MarchCall &, bool, const __VA_ARGS__ &);
+VT_FINISH(SumIO<1>)
+VT_FINISH(SumIO<2>)
+VT_FINISH(SumIO<3>)
+VT_FINISH(SumIO<4>)
+VT_FINISH(SumDynIO)
+VT_FINISH(ExtIO<true>)
+VT_FINISH(ExtIO<false>)
+VT_FINISH(VolIO)
+VT_FINISH(CountIO)
+VT_FINISH(SegIO)
+VT_FINISH(FillIO<SumDynIO>)
+VT_FINISH(FillIO<ExtIO<true>>)
+VT_FINISH(FillIO<ExtIO<false>>)
+VT_FINISH(FillIO<VolIO>)
+VT_FINISH(MarchRecordIO<SumIO<1>>)
+VT_FINISH(MarchRecordIO<SumDynIO>)
+VT_FINISH(MarchRecordIO<VolIO>)
+#undef VT_FINISH
+
+}  // namespace vt

@@ -4,9 +4,12 @@ The ray engine (vortrace_amd/csrc/engine.h) runs node steps every iteration
 and groups leaf steps and walk steps: a wave runs its leaf steps once
 ``leaf_batch`` of its lanes are at a leaf, and its walk steps once
 ``walk_batch`` lanes wait for one.  Rays are taken from ``ray_parts``
-partitions (8: one per XCD, for L2 locality; or 1).  Once a lane has no ray
-left to take, it walks an interval of a busy lane's ray of its wave, recording
-up to ``help_events`` boundaries of it (0: off).  Results never depend on
+partitions (8: one per XCD, for L2 locality; or 1).  With ``help_events`` > 0
+rays are marched over the cells' neighbour lists (march.hip), the lanes of a
+wave share the march's check (8 * ``help_events`` intervals at once), and the
+engine runs what the march leaves, its idle lanes walking intervals of busy
+lanes' rays (up to ``help_events`` boundaries each); 0 runs every ray in the
+engine, without help.  Results never depend on
 these values, only speed.  The kd-tree's leaf size stays the reference's 10
 (src/pointcloud.cpp:204): the order of equidistant neighbours, and with it the
 crossing sequences, depends on it.
