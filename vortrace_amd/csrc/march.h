@@ -49,15 +49,16 @@ struct MarchRays {
   uint32_t tile_row, tile_n;
 };
 
-// Work buffers of a march, [k][stride] with one column per batch slot.
+// Work buffers of a march, one row per batch slot.
 struct MarchBufs {
-  uint4 *seq;    // entry k: position where cell k is entered, cell | image, zone half-width
-  double *ins;   // where the recursion inserts cell k (periodic clouds)
-  // Per column: the entry to march from (kNone: not at all), then the number
+  // [slot][cap], entry k: position where cell k is entered, cell | image, zone
+  // half-width.
+  uint4 *seq;
+  // Per slot: the entry to march from (kNone: not at all), then the number
   // of cells (0: left to the engine).
   uint32_t *c0;
   uint32_t *ctr;  // kMarchCounters words: slots taken of each part of the queue
-  int cap, stride;
+  int cap;
 };
 
 constexpr int kMarchCounters = kParts;

@@ -91,7 +91,7 @@ __global__ __launch_bounds__(kBlock) void k_locate(DevCloud C, Scratch S, MarchR
         }
         code = image_code(im[0], im[1], im[2]);
       }
-      gst(B.seq + j, make_uint4(0u, 0u, c0 | (code << kNbSlotBits), 0u));
+      gst(B.seq + (size_t)j * B.cap, make_uint4(0u, 0u, c0 | (code << kNbSlotBits), 0u));
     }
     gst(B.c0 + j, ok ? 0u : kNone);
   }
@@ -287,7 +287,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
           double scale;
           M.delta = clearance(C, M.r, scale);
           zone_c = 1e-13 * scale;
-          const uint4 e = gld(B.seq + (size_t)k * B.stride + j);
+          const uint4 e = gld(B.seq + (size_t)j * B.cap + k);
           const uint32_t slot = e.z & kNbSlotMask;
           const int ic = (int)(e.z >> kNbSlotBits);
           const double2 xy = gld(reinterpret_cast<const double2 *>(C.gen + slot));
@@ -619,7 +619,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
           const uint32_t ic = PER ? image_code(M.im[0], M.im[1], M.im[2]) : kNbCentre;
           const uint64_t sb = (uint64_t)__double_as_longlong(sv);
           if (gl == 0)
-            gst(B.seq + (size_t)M.k * B.stride + j,
+            gst(B.seq + (size_t)j * B.cap + M.k,
                 make_uint4((uint32_t)sb, (uint32_t)(sb >> 32), n | (ic << kNbSlotBits),
                            __float_as_uint(zf)));
           M.enter(C, n, g, sv);
@@ -637,95 +637,38 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(3))) void k_
   if (lane == 0 && nball) atomicAdd(&stats->queries, (unsigned long long)nball);
 }
 
-// A ray's records start at the place its wave reserved for it.
-template <class IO>
-struct Finish {
-  using Sink = typename IO::Sink;
-  static __device__ __forceinline__ void reserve(const IO &, Sink &, int, int) {}
-  static __device__ __forceinline__ void begin(const IO &io, int64_t ray, Sink &sk) {
-    io.begin(ray, sk);
-  }
-  static __device__ __forceinline__ int end(const IO &io, int64_t ray, Sink &sk) {
-    return io.end(ray, sk);
-  }
-};
-template <class Inner>
-struct MarchRecSink : Inner::Sink {
-  RecPool pool;
-  unsigned long long next;
-  uint32_t ray;
-  __device__ __forceinline__ void seg(uint32_t cell, double a, double b) {
-    const uint32_t k = (uint32_t)this->n;
-    Inner::Sink::seg(cell, a, b);
-    if (next < pool.cap) {
-      SegRec *q = pool.rec + next;
-      gst_nt(reinterpret_cast<uint4 *>(q), make_uint4(cell, ray, k, 0u));
-      gst_nt(&q->ds, b - a);
-    } else {
-      atomicOr(pool.overflow, 1);
-    }
-    ++next;
-  }
-};
-template <class Inner>
-struct Finish<MarchRecordIO<Inner>> {
-  using IO = MarchRecordIO<Inner>;
-  using Sink = MarchRecSink<Inner>;
-  // The wave takes one run of whole chunks, its rays' records in lane order;
-  // the last lanes mark the rest of the last chunk unwritten.
-  static __device__ __forceinline__ void reserve(const IO &io, Sink &sk, int cells, int lane) {
-    int inc = cells;
-    for (int o = 1; o < 64; o <<= 1) {
-      const int v = __shfl_up(inc, o);
-      if (lane >= o) inc += v;
-    }
-    const int total = __shfl(inc, 63);
-    const int whole = (total + kRecChunk - 1) / kRecChunk * kRecChunk;
-    unsigned long long base = 0;
-    if (lane == 0 && whole) base = atomicAdd(io.pool.head, (unsigned long long)whole);
-    base = __shfl(base, 0);
-    sk.pool = io.pool;
-    sk.next = base + (unsigned long long)(inc - cells);
-    const unsigned long long rest = base + (unsigned long long)total + (unsigned long long)lane;
-    if (lane < whole - total && rest < io.pool.cap) gst(&io.pool.rec[rest].ray, kNone);
-  }
-  static __device__ __forceinline__ void begin(const IO &io, int64_t ray, Sink &sk) {
-    io.inner.begin(ray, static_cast<typename Inner::Sink &>(sk));
-    sk.ray = (uint32_t)ray;
-  }
-  static __device__ __forceinline__ int end(const IO &io, int64_t ray, Sink &sk) {
-    return io.inner.end(ray, static_cast<typename Inner::Sink &>(sk));
-  }
-};
+// Rays per wave of the replay, cells whose entries it holds in LDS (at least
+// the longest ray's), and intervals it can hold for its lanes.
+constexpr int kReplayRays = 4;
+constexpr int kReplayCells = 576;
+constexpr int kPool = 512;
 
-// Intervals a wave can hold for its lanes (64-bit items in LDS).
-constexpr int kPool = 1024;
-
-// The replay of the recursion (see march.h) over the lanes of a wave, then the
-// segments.  An item is an interval (i, j), j >= i + 2, of a ray's cells that
-// the recursion visits as a pair; its split point inserts a cell k between
-// them and leaves (i, k) and (k, j).  Intervals do not depend on one another,
-// so any lane takes any interval of the wave's rays: lanes without a ray, or
-// whose ray is done, work on the others'.  Bound by the latency of the entries'
-// reads, one column per ray (2.7 ms at 512^2 rays, 2M clustered cells).
-template <bool PER, class IO>
-__global__ __launch_bounds__(64) void k_finish(DevCloud C, MarchRays R, MarchBufs B, int rpw,
-                                               int pool, IO io, uint32_t *fall, ErrRec *err,
-                                               Stats *stats) {
+// The replay of the recursion (see march.h) over the lanes of a wave.  An item
+// is an interval (i, j), j >= i + 2, of a ray's cells that the recursion visits
+// as a pair; its split point inserts a cell k between them and leaves (i, k)
+// and (k, j).  Intervals do not depend on one another, so any lane takes any
+// interval of the wave's rays.  A ray's entries are one contiguous run, copied
+// to LDS first: the search for the split point's cell is a chain of reads, and
+// with the entries in device memory it took 2.7 of the 11.7 ms of a call (2M
+// clustered cells, 512^2 rays).  Four rays keep a wave's lanes busy (a ray has
+// one interval per cell) in 15 KB, so that ten waves share a CU.
+template <bool PER>
+__global__ __launch_bounds__(64) void k_replay(DevCloud C, MarchRays R, MarchBufs B, int room,
+                                               int pool, uint32_t *fall, Stats *stats) {
+  extern __shared__ uint4 dyn[];  // room entries, then where the recursion inserts them
+  uint4 *ent = dyn;
+  double *ins = reinterpret_cast<double *>(dyn + room);
   __shared__ uint64_t item[kPool];
-  __shared__ double geo[7][64];
-  __shared__ int cells[64];
-  __shared__ uint32_t bad[64];
+  __shared__ double geo[7][kReplayRays];
+  __shared__ int cells[kReplayRays], start[kReplayRays];
+  __shared__ uint32_t bad[kReplayRays];
   const int lane = threadIdx.x;
-  const int64_t blk = xcd_block(blockIdx.x, gridDim.x);
-  const int64_t j0 = blk * rpw;
+  const int64_t j0 = xcd_block(blockIdx.x, gridDim.x) * kReplayRays;
   const int64_t j = j0 + lane;
-  const bool mine = lane < rpw && j < R.n;
+  const bool mine = lane < kReplayRays && j < R.n;
   int K = 0;
   int64_t ray = 0;
   RayGeom r;
-  uint64_t first[2] = {0, 0};
-  int nfirst = 0;
   if (mine) {
     ray = march_ray(R, j);
     K = (int)gld(B.c0 + j);
@@ -737,28 +680,29 @@ __global__ __launch_bounds__(64) void k_finish(DevCloud C, MarchRays R, MarchBuf
     }
     geo[6][lane] = r.len;
   }
-  bool fail = mine && K == 0;
-  auto entry = [&](int64_t col, int k) { return gld(B.seq + (size_t)k * B.stride + col); };
+  if (lane < kReplayRays) {
+    cells[lane] = K;
+    bad[lane] = mine && K == 0 ? 1u : 0u;
+  }
+  __syncthreads();
   auto at = [](const uint4 &e) {
     return __longlong_as_double((long long)(((uint64_t)e.y << 32) | e.x));
   };
-  // The cell k of [lo, hi] that s falls in, clear of both its boundaries.
-  auto locate = [&](int64_t col, int n, double len, double s, int lo, int hi, uint4 &ek) {
-    ek = entry(col, lo);
-    if (s < at(ek)) return -1;
+  // The cell k of [lo, hi] that s falls in, clear of both its boundaries, of a
+  // ray of n cells from entry `e0`; -1: none.
+  auto locate = [&](int e0, int n, double len, double s, int lo, int hi) {
+    if (s < at(ent[e0 + lo])) return -1;
     while (hi > lo) {
       const int mid = (lo + hi + 1) >> 1;
-      const uint4 em = entry(col, mid);
-      if (at(em) <= s) {
+      if (at(ent[e0 + mid]) <= s)
         lo = mid;
-        ek = em;
-      } else {
+      else
         hi = mid - 1;
-      }
     }
+    const uint4 ek = ent[e0 + lo];
     double next = len, zn = 0.0;
     if (lo + 1 < n) {
-      const uint4 en = entry(col, lo + 1);
+      const uint4 en = ent[e0 + lo + 1];
       next = at(en);
       zn = (double)__uint_as_float(en.w);
     }
@@ -768,211 +712,290 @@ __global__ __launch_bounds__(64) void k_finish(DevCloud C, MarchRays R, MarchBuf
   auto pack = [](int owner, int depth, int i, int k) {
     return (uint64_t)owner | ((uint64_t)depth << 8) | ((uint64_t)i << 16) | ((uint64_t)k << 32);
   };
-  if (mine && K > 0) {
-    const uint32_t a = entry(j, 0).z & kNbSlotMask, b = entry(j, K - 1).z & kNbSlotMask;
-    if constexpr (PER) {
-      gst(B.ins + j, 0.0);
-      gst(B.ins + (size_t)(K - 1) * B.stride + j, r.len);
-      if (a == b) {
-        // Same cell at both ends: dyadic probes for another one
-        // (src/ray.cpp:220-246).
-        fail = true;
-        bool go = K > 1;
-        for (int lv = 1; go && lv <= 10; ++lv)
-          for (int i = 1; go && i < (1 << lv); i += 2) {
-            const double mid = r.len * i / (1 << lv);
-            uint4 ek;
-            const int k = locate(j, K, r.len, mid, 0, K - 1, ek);
-            if (k < 0) {
-              go = false;
-            } else if ((ek.z & kNbSlotMask) != a) {
-              go = false;
-              fail = false;
-              gst(B.ins + (size_t)k * B.stride + j, mid);
-              if (k >= 2) first[nfirst++] = pack(lane, 1, 0, k);
-              if (K - 1 - k >= 2) first[nfirst++] = pack(lane, 0, k, K - 1);
-            }
-          }
-      } else if (K >= 3) {
-        first[nfirst++] = pack(lane, 0, 0, K - 1);
-      }
-    } else {
-      fail = a == b && K > 1;
-      if (!fail && K >= 3) first[nfirst++] = pack(lane, 0, 0, K - 1);
-    }
-  }
-  cells[lane] = K;
-  bad[lane] = 0u;
-  __syncthreads();
-  int count = 0;
   uint32_t given = 0, back = 0;
-#pragma unroll
-  for (int q = 0; q < 2; ++q) {
-    const bool put = nfirst > q;
-    const uint64_t m = __ballot(put);
-    const int p = count + __popcll(m & ((1ull << lane) - 1ull));
-    if (put) {
-      if (p < pool) {
-        item[p] = first[q];
-      } else {
-        bad[lane] = 1u;
-        ++back;
-      }
-    }
-    count = min(pool, count + (int)__popcll(m));
-  }
-  __syncthreads();
-  while (count > 0) {
-    const int take = count < 64 ? count : 64;
-    count -= take;
-    uint64_t it = 0;
-    const bool work = lane < take;
-    if (work) it = item[count + lane];
+  for (int r0 = 0; r0 < kReplayRays;) {
+    // As many rays as fit, one at least (a ray has at most `room` cells).
+    int r1 = r0, held = 0;
+    while (r1 < kReplayRays && (r1 == r0 || held + cells[r1] <= room)) held += cells[r1++];
     __syncthreads();
-    uint64_t child[2] = {0, 0};
-    bool put[2] = {false, false};
-    int owner = 0;
-    if (work) {
-      owner = (int)(it & 255u);
-      const int depth = (int)((it >> 8) & 255u);
-      const int i = (int)((it >> 16) & 0xFFFFu), jj = (int)((it >> 32) & 0xFFFFu);
-      if (owner != lane) ++given;
-      if (!bad[owner]) {
-        const int64_t col = j0 + owner;
-        const int n = cells[owner];
-        RayGeom g;
-#pragma unroll
-        for (int d = 0; d < 3; ++d) {
-          g.a[d] = geo[d][owner];
-          g.d[d] = geo[3 + d][owner];
-        }
-        g.len = geo[6][owner];
-        const uint32_t ci = entry(col, i).z & kNbSlotMask, cj = entry(col, jj).z & kNbSlotMask;
-        bool ok = ci != cj && depth < 120;
-        double s = 0.0, p1[3], p2[3];
-        double sc = 0.0, sn = g.len;
-        if constexpr (PER) {
-          sc = gld(B.ins + (size_t)i * B.stride + col);
-          sn = gld(B.ins + (size_t)jj * B.stride + col);
-        }
-        bool analytic = split_point<PER>(C, g, ci, cj, sc, sn, s, p1, p2);
-        int k = -1;
-        uint4 ek;
-        if (ok && analytic) {
-          if constexpr (PER) {
-            const double l2 = sc + 1e-15, h2 = sn - 1e-15;
-            s = (s < l2) ? l2 : ((h2 < s) ? h2 : s);
-          }
-          k = locate(col, n, g.len, s, i, jj, ek);
-        } else if (PER && ok) {
-          // The reference's bisection between the two cells.
-          double lo = sc, hi = sn;
-          for (int q = 0; q < 64; ++q) {
-            const double mid = 0.5 * (lo + hi);
-            const int km = locate(col, n, g.len, mid, i, jj, ek);
-            if (km < 0) break;
-            const uint32_t cm = ek.z & kNbSlotMask;
-            if (cm != ci && cm != cj) {
-              const double l2 = sc + 1e-15, h2 = sn - 1e-15;
-              s = (mid < l2) ? l2 : ((h2 < mid) ? h2 : mid);
-              k = s == mid ? km : -1;
-              break;
-            }
-            if (cm == ci)
-              lo = mid;
-            else
-              hi = mid;
-            if (hi - lo < 1e-11) break;
-          }
-        }
-        if (k <= i || k >= jj) {
-          ok = false;
-        } else {
-          const uint32_t ck = ek.z & kNbSlotMask;
-          ok = ok && ck != ci && ck != cj;
-        }
-        if (!ok) {
-          bad[owner] = 1u;
-        } else {
-          if constexpr (PER) gst(B.ins + (size_t)k * B.stride + col, s);
-          put[0] = jj - k >= 2;
-          child[0] = pack(owner, depth, k, jj);
-          put[1] = k - i >= 2;
-          child[1] = pack(owner, depth + 1, i, k);
-        }
+    if (lane == 0) {
+      int at0 = 0;
+      for (int q = r0; q < r1; ++q) {
+        start[q] = at0;
+        at0 += cells[q];
       }
     }
-    // Insertion points written here are read by whichever lane takes the
-    // children.
-    __threadfence_block();
+    __syncthreads();
+    for (int q = r0; q < r1; ++q)
+      for (int k = lane; k < cells[q]; k += 64)
+        ent[start[q] + k] = gld(B.seq + (size_t)(j0 + q) * B.cap + k);
+    __syncthreads();
+    // The rays' first intervals, by their own lanes.
+    uint64_t first[2] = {0, 0};
+    int nfirst = 0;
+    if (lane >= r0 && lane < r1 && K > 0) {
+      const int e0 = start[lane];
+      const uint32_t a = ent[e0].z & kNbSlotMask, b = ent[e0 + K - 1].z & kNbSlotMask;
+      bool fail = false;
+      if constexpr (PER) {
+        ins[e0] = 0.0;
+        ins[e0 + K - 1] = r.len;
+        if (a == b) {
+          // Same cell at both ends: dyadic probes for another one
+          // (src/ray.cpp:220-246).
+          fail = true;
+          bool go = K > 1;
+          for (int lv = 1; go && lv <= 10; ++lv)
+            for (int i = 1; go && i < (1 << lv); i += 2) {
+              const double mid = r.len * i / (1 << lv);
+              const int k = locate(e0, K, r.len, mid, 0, K - 1);
+              if (k < 0) {
+                go = false;
+              } else if ((ent[e0 + k].z & kNbSlotMask) != a) {
+                go = false;
+                fail = false;
+                ins[e0 + k] = mid;
+                if (k >= 2) first[nfirst++] = pack(lane, 1, 0, k);
+                if (K - 1 - k >= 2) first[nfirst++] = pack(lane, 0, k, K - 1);
+              }
+            }
+        } else if (K >= 3) {
+          first[nfirst++] = pack(lane, 0, 0, K - 1);
+        }
+      } else {
+        fail = a == b && K > 1;
+        if (!fail && K >= 3) first[nfirst++] = pack(lane, 0, 0, K - 1);
+      }
+      if (fail) bad[lane] = 1u;
+    }
+    int count = 0;
 #pragma unroll
     for (int q = 0; q < 2; ++q) {
-      const uint64_t m = __ballot(put[q]);
+      const bool put = nfirst > q;
+      const uint64_t m = __ballot(put);
       const int p = count + __popcll(m & ((1ull << lane) - 1ull));
-      if (put[q]) {
+      if (put) {
         if (p < pool) {
-          item[p] = child[q];
+          item[p] = first[q];
         } else {
-          bad[owner] = 1u;  // no room: the engine walks the ray
+          bad[lane] = 1u;
           ++back;
         }
       }
       count = min(pool, count + (int)__popcll(m));
     }
     __syncthreads();
-  }
-  fail |= mine && bad[lane] != 0u;
-  const int out = mine && !fail ? K : 0;
-  using F = Finish<IO>;
-  typename F::Sink sk;
-  F::reserve(io, sk, out, lane);
-  if (out > 0) {
-    F::begin(io, ray, sk);
-    uint4 e = entry(j, 0);
-    for (int k = 0; k < out; ++k) {
-      uint4 nx = e;
-      double b = r.len;
-      if (k + 1 < out) {
-        nx = entry(j, k + 1);
-        b = at(nx);
+    while (count > 0) {
+      const int take = count < 64 ? count : 64;
+      count -= take;
+      uint64_t it = 0;
+      const bool work = lane < take;
+      if (work) it = item[count + lane];
+      __syncthreads();
+      uint64_t child[2] = {0, 0};
+      bool put[2] = {false, false};
+      int owner = 0;
+      if (work) {
+        owner = (int)(it & 255u);
+        const int depth = (int)((it >> 8) & 255u);
+        const int i = (int)((it >> 16) & 0xFFFFu), jj = (int)((it >> 32) & 0xFFFFu);
+        if (owner != lane) ++given;
+        if (!bad[owner]) {
+          const int e0 = start[owner], n = cells[owner];
+          RayGeom g;
+#pragma unroll
+          for (int d = 0; d < 3; ++d) {
+            g.a[d] = geo[d][owner];
+            g.d[d] = geo[3 + d][owner];
+          }
+          g.len = geo[6][owner];
+          const uint32_t ci = ent[e0 + i].z & kNbSlotMask, cj = ent[e0 + jj].z & kNbSlotMask;
+          bool ok = ci != cj && depth < 120;
+          double s = 0.0, p1[3], p2[3];
+          double sc = 0.0, sn = g.len;
+          if constexpr (PER) {
+            sc = ins[e0 + i];
+            sn = ins[e0 + jj];
+          }
+          const bool analytic = split_point<PER>(C, g, ci, cj, sc, sn, s, p1, p2);
+          int k = -1;
+          if (ok && analytic) {
+            if constexpr (PER) {
+              const double l2 = sc + 1e-15, h2 = sn - 1e-15;
+              s = (s < l2) ? l2 : ((h2 < s) ? h2 : s);
+            }
+            k = locate(e0, n, g.len, s, i, jj);
+          } else if (PER && ok) {
+            // The reference's bisection between the two cells.
+            double lo = sc, hi = sn;
+            for (int q = 0; q < 64; ++q) {
+              const double mid = 0.5 * (lo + hi);
+              const int km = locate(e0, n, g.len, mid, i, jj);
+              if (km < 0) break;
+              const uint32_t cm = ent[e0 + km].z & kNbSlotMask;
+              if (cm != ci && cm != cj) {
+                const double l2 = sc + 1e-15, h2 = sn - 1e-15;
+                s = (mid < l2) ? l2 : ((h2 < mid) ? h2 : mid);
+                k = s == mid ? km : -1;
+                break;
+              }
+              if (cm == ci)
+                lo = mid;
+              else
+                hi = mid;
+              if (hi - lo < 1e-11) break;
+            }
+          }
+          if (k <= i || k >= jj) {
+            ok = false;
+          } else {
+            const uint32_t ck = ent[e0 + k].z & kNbSlotMask;
+            ok = ok && ck != ci && ck != cj;
+          }
+          if (!ok) {
+            bad[owner] = 1u;
+          } else {
+            if constexpr (PER) ins[e0 + k] = s;
+            put[0] = jj - k >= 2;
+            child[0] = pack(owner, depth, k, jj);
+            put[1] = k - i >= 2;
+            child[1] = pack(owner, depth + 1, i, k);
+          }
+        }
       }
-      sk.seg(e.z & kNbSlotMask, at(e), b);
-      e = nx;
+#pragma unroll
+      for (int q = 0; q < 2; ++q) {
+        const uint64_t m = __ballot(put[q]);
+        const int p = count + __popcll(m & ((1ull << lane) - 1ull));
+        if (put[q]) {
+          if (p < pool) {
+            item[p] = child[q];
+          } else {
+            bad[owner] = 1u;  // no room: the engine walks the ray
+            ++back;
+          }
+        }
+        count = min(pool, count + (int)__popcll(m));
+      }
+      __syncthreads();
     }
-    const int rc = F::end(io, ray, sk);
-    if (rc) report_error(err, rc, ray, 0.0, 0.0, 0.0, 0u, 0u);
-  } else if (fail) {
+    r0 = r1;
+  }
+  if (mine && bad[lane]) {
+    if (K) gst(B.c0 + j, 0u);
     const unsigned long long q = atomicAdd(&stats->fallback, 1ull);
     gst(fall + q, (uint32_t)ray);
   }
-  uint64_t seg = (uint64_t)out;
   for (int o = 32; o; o >>= 1) {
-    seg += __shfl_xor(seg, o);
     given += __shfl_xor(given, o);
     back += __shfl_xor(back, o);
   }
   if (lane == 0) {
-    atomicAdd(&stats->segments, (unsigned long long)seg);
     if (given) atomicAdd(&stats->intervals, (unsigned long long)given);
     if (back) atomicAdd(&stats->intervals_back, (unsigned long long)back);
   }
 }
 
+// The IO that takes a lane's segments, and the record pool when there is one.
+template <class IO>
+struct Emit {
+  using Inner = IO;
+  static constexpr bool kRecord = false;
+  static __device__ __forceinline__ const IO &inner(const IO &io) { return io; }
+};
+template <class I>
+struct Emit<MarchRecordIO<I>> {
+  using Inner = I;
+  static constexpr bool kRecord = true;
+  static __device__ __forceinline__ const I &inner(const MarchRecordIO<I> &io) { return io.inner; }
+};
+
+// Hands the segments of the batch's rays to the sinks, one ray per lane; with
+// records, the wave then writes them ray by ray, its lanes along the ray, so
+// that a ray's records are one run of whole lines (a lane writing its own ray's
+// took 2.4 ms more at 2M cells, 512^2 rays).
+template <class IO>
+__global__ __launch_bounds__(64) void k_emit(MarchRays R, MarchBufs B, IO io, ErrRec *err,
+                                             Stats *stats) {
+  const int lane = threadIdx.x;
+  const int64_t j0 = xcd_block(blockIdx.x, gridDim.x) * 64;
+  const int64_t j = j0 + lane;
+  const bool mine = j < R.n;
+  const int K = mine ? (int)gld(B.c0 + j) : 0;
+  const uint4 *ent = B.seq + (size_t)(mine ? j : 0) * B.cap;
+  auto at = [](const uint4 &e) {
+    return __longlong_as_double((long long)(((uint64_t)e.y << 32) | e.x));
+  };
+  int64_t ray = 0;
+  double len = 0.0;
+  if (K > 0) {
+    ray = march_ray(R, j);
+    RayGeom r;
+    make_ray(R.start + 3 * ray, R.end + 3 * ray, r);
+    len = r.len;
+    const auto &in = Emit<IO>::inner(io);
+    typename Emit<IO>::Inner::Sink sk;
+    in.begin(ray, sk);
+    // Four segments at a time, their reads in flight together.
+    uint4 e = gld(ent);
+    int k = 0;
+    for (; k + 4 < K; k += 4) {
+      uint4 n[4];
+#pragma unroll
+      for (int i = 0; i < 4; ++i) n[i] = gld(ent + k + 1 + i);
+      sk.seg(e.z & kNbSlotMask, at(e), at(n[0]));
+#pragma unroll
+      for (int i = 0; i < 3; ++i) sk.seg(n[i].z & kNbSlotMask, at(n[i]), at(n[i + 1]));
+      e = n[3];
+    }
+    for (; k < K; ++k) {
+      uint4 n = e;
+      double b = len;
+      if (k + 1 < K) {
+        n = gld(ent + k + 1);
+        b = at(n);
+      }
+      sk.seg(e.z & kNbSlotMask, at(e), b);
+      e = n;
+    }
+    const int rc = in.end(ray, sk);
+    if (rc) report_error(err, rc, ray, 0.0, 0.0, 0.0, 0u, 0u);
+  }
+  int inc = K;
+  for (int o = 1; o < 64; o <<= 1) {
+    const int v = __shfl_up(inc, o);
+    if (lane >= o) inc += v;
+  }
+  const int total = __shfl(inc, 63);
+  if (lane == 0 && total) atomicAdd(&stats->segments, (unsigned long long)total);
+  if constexpr (Emit<IO>::kRecord) {
+    // One run of whole chunks; the rest of the last one is marked unwritten.
+    const int whole = (total + kRecChunk - 1) / kRecChunk * kRecChunk;
+    unsigned long long base = 0;
+    if (lane == 0 && whole) base = atomicAdd(io.pool.head, (unsigned long long)whole);
+    base = __shfl(base, 0);
+    if (base + (unsigned long long)whole > io.pool.cap) {
+      if (lane == 0) atomicOr(io.pool.overflow, 1);
+      return;
+    }
+    if (lane < whole - total) gst(&io.pool.rec[base + total + lane].ray, kNone);
+    for (int q = 0; q < 64; ++q) {
+      const int n = __shfl(K, q), off = __shfl(inc, q) - n;
+      const uint32_t id = (uint32_t)__shfl((int)ray, q);
+      const double end = __shfl(len, q);
+      const uint4 *src = B.seq + (size_t)(j0 + q) * B.cap;
+      for (int k = lane; k < n; k += 64) {
+        const uint4 e = gld(src + k);
+        const double b = k + 1 < n ? at(gld(src + k + 1)) : end;
+        SegRec *o = io.pool.rec + base + off + k;
+        gst_nt(reinterpret_cast<uint4 *>(o), make_uint4(e.z & kNbSlotMask, id, (uint32_t)k, 0u));
+        gst_nt(&o->ds, b - at(e));
+      }
+    }
+  }
+}
+
 }  // namespace
-
-// Rays a wave marches: all its lanes' when there are rays for every SIMD, else
-// fewer, so that the rays spread over the chip.
-int march_rays_per_wave(int64_t n, int cus) {
-  int rpw = 64;
-  while (rpw > 4 && (n + rpw - 1) / rpw < 8ll * cus) rpw >>= 1;
-  return rpw;
-}
-
-// Waves of a batch: a multiple of kParts, so that every XCD has the same share.
-int64_t march_waves(int64_t n, int cus) {
-  const int rpw = march_rays_per_wave(n, cus);
-  return ((n + rpw - 1) / rpw + kParts - 1) / kParts * kParts;
-}
 
 void march_build_lists(const DevCloud &C, uint32_t *nb, float *r2, hipStream_t st) {
   const unsigned grid = (C.n + kNbWindow - 1) / kNbWindow;
@@ -1015,15 +1038,19 @@ void march_batch(const MarchCall &m, bool periodic) {
 
 template <class IO>
 void march_finish(const MarchCall &m, bool periodic, const IO &io) {
-  const int rpw = march_rays_per_wave(m.R.n, m.cus);
-  const int64_t nb = march_waves(m.R.n, m.cus);
+  auto waves = [&](int64_t rays) {
+    return (unsigned)(((m.R.n + rays - 1) / rays + kParts - 1) / kParts * kParts);
+  };
+  const int room = std::max(kReplayCells, m.B.cap);
+  const size_t lds = (size_t)room * (sizeof(uint4) + (periodic ? sizeof(double) : 0));
   const int pool = std::min(m.pool, kPool);
   if (periodic)
-    k_finish<true, IO><<<(unsigned)nb, 64, 0, m.st>>>(m.C, m.R, m.B, rpw, pool, io, m.fall, m.err,
-                                                      m.stats);
+    k_replay<true><<<waves(kReplayRays), 64, lds, m.st>>>(m.C, m.R, m.B, room, pool, m.fall,
+                                                          m.stats);
   else
-    k_finish<false, IO><<<(unsigned)nb, 64, 0, m.st>>>(m.C, m.R, m.B, rpw, pool, io, m.fall, m.err,
-                                                       m.stats);
+    k_replay<false><<<waves(kReplayRays), 64, lds, m.st>>>(m.C, m.R, m.B, room, pool, m.fall,
+                                                           m.stats);
+  k_emit<IO><<<waves(64), 64, 0, m.st>>>(m.R, m.B, io, m.err, m.stats);
 }
 
 #define VT_FINISH(...) template void march_finish<__VA_ARGS__>(const MarchCall &, bool, const __VA_ARGS__ &);

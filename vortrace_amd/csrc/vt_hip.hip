@@ -357,7 +357,7 @@ struct vt_cloud {
   uint32_t *d_nb = nullptr;     // neighbour lists (null: every ray runs in the engine)
   float *d_nr2 = nullptr;
   BNode *d_boxes = nullptr;     // and the tree's boxes
-  MarchBufs march{};            // the march's work buffers, for march_rays columns
+  MarchBufs march{};            // the march's work buffers, for march_rays slots
   size_t march_rays = 0;
   uint32_t *d_fall = nullptr;   // rays the march left to the engine
   size_t fall_cap = 0;
@@ -375,7 +375,7 @@ struct vt_cloud {
                     (void *)scratch.walk_tag, (void *)scratch.walk_s,
                     (void *)scratch.big_id, (void *)scratch.big_d, (void *)help_ev,
                     (void *)help_steal, (void *)d_defer, (void *)d_nb, (void *)d_nr2,
-                    (void *)march.seq, (void *)march.ins, (void *)march.c0, (void *)d_boxes,
+                    (void *)march.seq, (void *)march.c0, (void *)d_boxes,
                     (void *)march.ctr, (void *)d_fall,
                     (void *)d_order, (void *)d_order_hist, (void *)d_order_grid})
       if (p) (void)hipFree(p);
@@ -712,20 +712,17 @@ int64_t ensure_march(vt_cloud *c, int64_t n) {
   // box diagonal; longer rays run in the engine.
   int cap = (int)(2.6 * std::cbrt((double)c->n)) + 64;
   cap = std::min(4096, std::max(128, (cap + 63) / 64 * 64));
-  const size_t per = (size_t)cap * (sizeof(uint4) + (c->periodic ? sizeof(double) : 0));
+  const size_t per = (size_t)cap * sizeof(uint4);
   const int64_t most = (int64_t)(kMarchBytes / per) / 64 * 64;
   const int64_t batches = (n + most - 1) / most;
   const int64_t rays = ((n + batches - 1) / batches + 63) / 64 * 64;
   if (c->march_rays < (size_t)rays || c->march.cap != cap) {
-    for (void *p : {(void *)c->march.seq, (void *)c->march.ins, (void *)c->march.c0,
-                    (void *)c->march.ctr})
+    for (void *p : {(void *)c->march.seq, (void *)c->march.c0, (void *)c->march.ctr})
       if (p) (void)hipFree(p);
     c->march = MarchBufs{};
     c->march_rays = 0;
     c->march.cap = cap;
-    c->march.stride = (int)rays;
     c->march.seq = dev_alloc<uint4>((size_t)cap * rays);
-    if (c->periodic) c->march.ins = dev_alloc<double>((size_t)cap * rays);
     c->march.c0 = dev_alloc<uint32_t>((size_t)rays);
     c->march.ctr = dev_alloc<uint32_t>(kMarchCounters);
     c->march_rays = (size_t)rays;
