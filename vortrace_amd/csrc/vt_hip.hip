@@ -897,6 +897,32 @@ __device__ __forceinline__ double pixel_centre(double lo, double hi, int64_t n, 
 // at (x_i, y_j, bounds[1]); with a rotation, p -> R (p - c) + c where
 // numpy.dot(p - c, R.T) evaluates each row as fma(p2, R_k2, fma(p1, R_k1,
 // p0 * R_k0)) (OpenBLAS' x86-64 kernels behind numpy).
+__device__ __forceinline__ void grid_ray(const vt_view &v, int64_t local, int64_t r, double *start,
+                                         double *end) {
+  const int64_t ny = v.ny;
+  const int64_t i = local / ny, j = local - i * ny;
+  const double x = pixel_centre(v.extent[0], v.extent[1], v.nx, i);
+  const double y = pixel_centre(v.extent[2], v.extent[3], ny, j);
+  double p[2][3] = {{x, y, v.bounds[0]}, {x, y, v.bounds[1]}};
+  if (v.rotate) {
+#pragma unroll
+    for (int e = 0; e < 2; ++e) {
+      const double a0 = p[e][0] - v.center[0], a1 = p[e][1] - v.center[1],
+                   a2 = p[e][2] - v.center[2];
+#pragma unroll
+      for (int k = 0; k < 3; ++k) {
+        const double *R = v.rot + 3 * k;
+        p[e][k] = __fma_rn(a2, R[2], __fma_rn(a1, R[1], a0 * R[0])) + v.center[k];
+      }
+    }
+  }
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    gst(start + 3 * r + k, p[0][k]);
+    gst(end + 3 * r + k, p[1][k]);
+  }
+}
+
 __global__ void k_grid_rays(const vt_view *views, const int64_t *offsets, int nviews,
                             int64_t nrays, double *start, double *end) {
   const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
@@ -906,30 +932,13 @@ __global__ void k_grid_rays(const vt_view *views, const int64_t *offsets, int nv
     const int mid = (lo + hi + 1) >> 1;
     if (gld(offsets + mid) <= r) lo = mid; else hi = mid - 1;
   }
-  const vt_view *v = views + lo;
-  const int64_t local = r - gld(offsets + lo);
-  const int64_t ny = v->ny;
-  const int64_t i = local / ny, j = local - i * ny;
-  const double x = pixel_centre(v->extent[0], v->extent[1], v->nx, i);
-  const double y = pixel_centre(v->extent[2], v->extent[3], ny, j);
-  double p[2][3] = {{x, y, v->bounds[0]}, {x, y, v->bounds[1]}};
-  if (v->rotate) {
-#pragma unroll
-    for (int e = 0; e < 2; ++e) {
-      const double a0 = p[e][0] - v->center[0], a1 = p[e][1] - v->center[1],
-                   a2 = p[e][2] - v->center[2];
-#pragma unroll
-      for (int k = 0; k < 3; ++k) {
-        const double *R = v->rot + 3 * k;
-        p[e][k] = __fma_rn(a2, R[2], __fma_rn(a1, R[1], a0 * R[0])) + v->center[k];
-      }
-    }
-  }
-#pragma unroll
-  for (int k = 0; k < 3; ++k) {
-    gst(start + 3 * r + k, p[0][k]);
-    gst(end + 3 * r + k, p[1][k]);
-  }
+  grid_ray(views[lo], r - gld(offsets + lo), r, start, end);
+}
+
+// One view, passed by value: no table to allocate and copy.
+__global__ void k_grid_rays_one(vt_view view, int64_t nrays, double *start, double *end) {
+  const int64_t r = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (r < nrays) grid_ray(view, r, r, start, end);
 }
 
 }  // namespace vt
@@ -2097,6 +2106,12 @@ int vt_grid_rays(const vt_view *views, size_t nviews, double *d_start, double *d
     if (!d_start || !d_end) return fail(VT_EINVAL, "null argument");
     if (nviews > (size_t)INT32_MAX) return fail(VT_EINVAL, "too many views");
     hipStream_t st = static_cast<hipStream_t>(stream);
+    if (nviews == 1) {
+      k_grid_rays_one<<<(unsigned)((n + 255) / 256), 256, 0, st>>>(views[0], n, d_start, d_end);
+      HIP_OK(hipGetLastError());
+      HIP_OK(hipStreamSynchronize(st));
+      return VT_OK;
+    }
     DevBufs B;
     vt_view *dv = B.get<vt_view>(nviews);
     int64_t *doff = B.get<int64_t>(nviews + 1);

@@ -136,17 +136,58 @@ def view_params(extent: ArrayLike, nres, bounds: ArrayLike,
     return v
 
 
+def device_view(extent: ArrayLike, nres, bounds: ArrayLike,
+                center: ArrayLike | None = None, *, proj: str | None = None,
+                yaw: float = 0., pitch: float = 0., roll: float = 0.):
+    """view_params of a grid the device builds with generate_projection_grid's
+    bits, or None: arguments it takes otherwise, or raises for, stay with it.
+    Rotated grids do too -- numpy.dot's evaluation order is the host BLAS's --
+    unless the rotation is the identity, whose products and sums are exact."""
+    if center is not None:
+        if proj is not None:
+            yaw, pitch, roll, _ = _plane_angles(proj)
+        if not np.array_equal(rotation_matrix(yaw, pitch, roll), np.eye(3)):
+            return None
+        c = np.asarray(center)
+        if c.shape != (3,) or c.dtype.kind not in "iuf" or not np.all(np.isfinite(c)):
+            return None
+    ext = np.asarray(extent)
+    if ext.shape not in ((2,), (2, 2)) or (ext.dtype != np.float64 and ext.dtype.kind not in "iu"):
+        return None
+    if not np.all(np.abs(ext.astype(np.float64)) < 2.0 ** 52):
+        return None
+    if isinstance(nres, int):
+        n = (nres, nres)
+    elif isinstance(nres, (tuple, list)) and len(nres) == 2:
+        n = nres
+    else:
+        return None
+    if not all(isinstance(k, (int, np.integer)) and not isinstance(k, bool) and 1 <= k < 2 ** 15
+               for k in n):
+        return None
+    b = np.asarray(bounds)
+    if b.shape != (2,) or b.dtype.kind not in "iuf" or not np.all(np.isfinite(b)):
+        return None
+    return view_params(extent, nres, bounds, center, proj=proj, yaw=yaw, pitch=pitch, roll=roll)
+
+
 def generate_projection_grids_device(views, device=None):
     """generate_projection_grid for many views at once on the device
     (vt_grid_rays).  `views` is a list of dicts of generate_projection_grid's
     arguments.  Returns (start, end, sizes): (R, 3) float64 device tensors
     holding every view's rays in turn (view v's ray i * ny + j is its pixel
     (i, j)) and the rays per view."""
+    import torch
+    dev = torch.device(device) if device is not None else torch.device("cuda")
+    recs = [view_params(**v) for v in views]
+    return _rays_of(recs, dev)
+
+
+def _rays_of(recs, dev):
+    """(start, end, sizes) of view records, on the device."""
     import ctypes as C
     import torch
     from . import _lib
-    dev = torch.device(device) if device is not None else torch.device("cuda")
-    recs = [view_params(**v) for v in views]
     sizes = [int(r.nx * r.ny) for r in recs]
     n = sum(sizes)
     start = torch.empty((n, 3), dtype=torch.float64, device=dev)

