@@ -96,6 +96,28 @@ def test_ray_counts(tuning, rays):
     np.testing.assert_array_equal(got[-1][0][:k], oc.project(s[:k], e[:k])[:, 0])
 
 
+@pytest.mark.parametrize("periodic,rays", [(False, 16_383), (False, 16_384), (False, 65_535),
+                                           (False, 65_536), (True, 16_384), (True, 196_607),
+                                           (True, 196_608)])
+def test_lanes_per_ray(tuning, periodic, rays):
+    """Ray counts on both sides of each change of a ray's lanes (256 CUs)."""
+    rng = np.random.default_rng(rays)
+    pos = rng.uniform(0, 1, (3000, 3))
+    if not periodic:
+        pos[:700] = rng.normal(0.4, 0.003, (700, 3))
+    pc = _cloud(pos, 1.0, periodic)
+    s, e = _chords(rays, 7, 0.0, 1.0)
+    if periodic:  # views, 0.9 of the box deep: oblique chords may have no unique split point
+        s[:, 2] = 0.05
+        e[:] = s + [0.0, 0.0, 0.9]
+    got = []
+    for he in (0, 128):
+        vt.tuning.set_tuning(help_events=he)
+        _say(f"  {rays} rays, periodic {periodic}, help_events {he}")
+        got.append(pc.projection(s, e))
+    np.testing.assert_array_equal(got[0], got[1])
+
+
 @pytest.mark.parametrize("periodic", [False, True])
 def test_clump_beside_void(tuning, periodic):
     """Lists full of a clump's generators do not reach across the void."""
