@@ -298,8 +298,9 @@ struct Marcher {
   }
 };
 
-// References of nodes still to be searched for an exit, per group, in LDS.
-constexpr int kBallStack = 112;
+// References of nodes still to be searched for an exit, per group, in LDS (a
+// step pushes up to two per lane).
+constexpr int ball_stack(int G) { return G == 4 ? 112 : (G == 8 ? 192 : 384); }
 
 // At most the squared distance from q to a box; q is the nearest float of a
 // point, which lies within `eps` of it along every axis.
@@ -343,6 +344,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 4 ? 3 :
   constexpr int kRays = 64 / G;
   // Generators of a leaf whose loads are in flight together.
   constexpr int kSearchChunk = G == 4 ? 5 : 3;
+  constexpr int kBallStack = ball_stack(G);
   __shared__ uint32_t stack_all[kRays * kBallStack];
   __shared__ Held held[kRays];
   __shared__ Images im;
@@ -723,13 +725,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 4 ? 3 :
       // nearest to every point of the two cells' chords, so cells and their
       // distances stay a fifth of the box.
       uint32_t name = M.b.n1;
-      if (!((double)M.b.t1 <= M.tend * (1.0 + kKeyTol))) {
-        // The ray ends in this cell, clear of its entry and of every exit.
-        const double v2 = M.r2_at(M.tend);
-        if (M.tend > (double)M.h->tent && M.tend < far && v2 < far * far &&
-            (lim == INFINITY || M.clear_of((double)lim, v2)))
-          cells = M.h->k + 1;
-      } else {
+      bool ends = !((double)M.b.t1 <= M.tend * (1.0 + kKeyTol));
+      if (!ends) {
         list = name & kNbSlotMask;
         read_ids(0);
         complete = gld(N.r2 + list);
@@ -737,8 +734,8 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 4 ? 3 :
         M.load(C, name, g);
         M.apart(g, name, e);
         double exit = M.exit_of(e, h, slack);
-        bool ok = true;
-        if (exit >= (double)M.b.t2 * (1.0 - kKeyTol)) {
+        bool ok = exit < M.tend;
+        if (fmin(exit, M.tend) >= (double)M.b.t2 * (1.0 - kKeyTol)) {
           // The keys cannot tell which of two is first.
           double g2[3], e2[3], h2, slack2;
           M.load(C, M.b.n2, g2);
@@ -754,10 +751,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 4 ? 3 :
             slack = slack2;
 #pragma unroll
             for (int d = 0; d < 3; ++d) g[d] = g2[d];
+            ok = exit < M.tend;
           } else {
-            ok = exit < exit2 - slack2;
+            ok = ok && exit < exit2 - slack2;
           }
           ok &= exit < (double)M.b.t3 * (1.0 - kKeyTol);
+        } else {
+          ends = exit - slack > M.tend;
         }
         const uint32_t n = list, rc = name >> kNbSlotBits;
         const double v2 = M.r2_at(exit);
@@ -778,7 +778,7 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 4 ? 3 :
         const float tent = M.h->tent;
         const int k = M.h->k + 1;
         const double chord = sv - M.h->s;
-        ok &= exit < M.tend && h > 1e-10 && fabs(chord - exit) <= zone &&
+        ok &= h > 1e-10 && fabs(chord - exit) <= zone &&
               chord > (double)tent + zone && chord < far && v2 < far * far && n != M.c &&
               k < B.cap && (lim == INFINITY || M.clear_of((double)lim, v2));
         if (ok) {
@@ -796,6 +796,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 4 ? 3 :
           ph = kMpScan;
           done = false;
         }
+      }
+      if (ends) {
+        // The ray ends in this cell, clear of its entry and of every exit.
+        const double v2 = M.r2_at(M.tend);
+        if (M.tend > (double)M.h->tent && M.tend < far && v2 < far * far &&
+            (lim == INFINITY || M.clear_of((double)lim, v2)))
+          cells = M.h->k + 1;
       }
       if (done) {
         if (gl == 0) gst(B.c0 + M.h->j, (uint32_t)cells);

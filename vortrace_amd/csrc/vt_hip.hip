@@ -155,6 +155,8 @@ __global__ __launch_bounds__(kBlock) void k_count(DevCloud C, Scratch S, const d
   run_rays<PER, EXP, HELP>(C, S, start, end, nrays, ray_list, defer, err, stats, io);
 }
 
+// k_fill and k_segs help always: they run a march's leftovers, where one ray of
+// 300 cells on one lane takes 20 ms.
 template <int MODE, bool PER, bool EXP>
 __global__ __launch_bounds__(kBlock) void k_fill(DevCloud C, Scratch S, const double *start,
                                                  const double *end, int64_t nrays,
@@ -166,14 +168,14 @@ __global__ __launch_bounds__(kBlock) void k_fill(DevCloud C, Scratch S, const do
   if constexpr (MODE == VT_SUM) {
     FillIO<SumDynIO> io{SumDynIO{C.fields, (int)C.nf, out, nout, nullptr}, offsets, slot_id, ids,
                         se, sx};
-    run_rays<PER, EXP>(C, S, start, end, nrays, ray_list, defer, err, stats, io);
+    run_rays<PER, EXP, !EXP>(C, S, start, end, nrays, ray_list, defer, err, stats, io);
   } else if constexpr (MODE == VT_MAX || MODE == VT_MIN) {
     FillIO<ExtIO<MODE == VT_MAX>> io{ExtIO<MODE == VT_MAX>{C.fields, (int)C.nf, out, nout, nullptr},
                                      offsets, slot_id, ids, se, sx};
-    run_rays<PER, EXP>(C, S, start, end, nrays, ray_list, defer, err, stats, io);
+    run_rays<PER, EXP, !EXP>(C, S, start, end, nrays, ray_list, defer, err, stats, io);
   } else {
     FillIO<VolIO> io{VolIO{C.fields, out, nout, nullptr}, offsets, slot_id, ids, se, sx};
-    run_rays<PER, EXP>(C, S, start, end, nrays, ray_list, defer, err, stats, io);
+    run_rays<PER, EXP, !EXP>(C, S, start, end, nrays, ray_list, defer, err, stats, io);
   }
 }
 
@@ -184,7 +186,7 @@ __global__ __launch_bounds__(kBlock) void k_segs(DevCloud C, Scratch S, const do
                                                  const int64_t *offsets, uint32_t *slot,
                                                  double *ds, ErrRec *err, Stats *stats) {
   SegIO io{offsets, slot, ds};
-  run_rays<PER, EXP>(C, S, start, end, nrays, ray_list, defer, err, stats, io);
+  run_rays<PER, EXP, !EXP>(C, S, start, end, nrays, ray_list, defer, err, stats, io);
 }
 
 template <int K, bool PER>
@@ -692,8 +694,21 @@ void launch(vt_cloud *c, K kernel, int64_t n, hipStream_t st, Timer &tm, A... ar
   c->scratch.help_depth = n < lanes ? 1 : 3;
   c->scratch.tile_row = c->ray_row;
   c->scratch.ray_order = (c->order_n == n && n > 0) ? c->d_order : nullptr;
+  Scratch s = c->scratch;
+  int blocks = grid;
+  if (n > 0 && n < grid && s.help_ev) {
+    // A few rays (a march's leftovers): a workgroup each, which share the
+    // interval buffers of all lanes.  A gift of more cells than its walker has
+    // room for is walked twice, and again by every giver above: of a ray of 358
+    // cells in 128-event buffers, 5,500 queries instead of 717.
+    blocks = (int)n;
+    s.lanes = blocks * kBlock;
+    const size_t more = c->scratch_lanes / (size_t)s.lanes;
+    s.help_cap = (int)std::min<size_t>(kHsMaxEvents, s.help_cap * more);
+    s.help_steal_cap = (int)std::min<size_t>(256, s.help_steal_cap * more);
+  }
   HIP_OK(hipEventRecord(tm.e0, st));
-  kernel<<<grid, kBlock, 0, st>>>(c->dc, c->scratch, args...);
+  kernel<<<blocks, kBlock, 0, st>>>(c->dc, s, args...);
   HIP_OK(hipGetLastError());
   HIP_OK(hipEventRecord(tm.e1, st));
 }
@@ -1686,25 +1701,23 @@ int vt_project_count(const vt_cloud *cc, const double *d_start, const double *d_
     hipStream_t st = static_cast<hipStream_t>(stream);
     if (nrays == 0) return VT_OK;
     const int64_t n = (int64_t)nrays;
-    auto go = [&](auto kfast, auto kslow) {
+    auto go = [&](auto kfast, auto khelp, auto kslow) {
       return march_then(
           c, d_start, d_end, n, CountIO{d_counts}, st,
           [&](Timer &tm, const uint32_t *list, int64_t nr) {
-            launch(c, kfast, nr, st, tm, d_start, d_end, nr, list, c->d_defer, d_counts,
-                   c->d_err, c->d_stats);
+            const bool help =
+                help_pays(VT_SUM, nr, grid_for(k_count<false, false>, INT64_MAX / 2, c->device));
+            launch(c, help ? khelp : kfast, nr, st, tm, d_start, d_end, nr, list, c->d_defer,
+                   d_counts, c->d_err, c->d_stats);
           },
           [&](Timer &tm, int64_t nd) {
             launch(c, kslow, nd, st, tm, d_start, d_end, nd, (const uint32_t *)c->d_defer,
                    (uint32_t *)nullptr, d_counts, c->d_err, c->d_stats);
           });
     };
-    const bool help = help_pays(VT_SUM, n, grid_for(k_count<false, false>, INT64_MAX / 2,
-                                                    c->device));
-    if (c->periodic)
-      return help ? go(k_count<true, false, true>, k_count<true, true>)
-                  : go(k_count<true, false>, k_count<true, true>);
-    return help ? go(k_count<false, false, true>, k_count<false, true>)
-                : go(k_count<false, false>, k_count<false, true>);
+    return c->periodic ? go(k_count<true, false>, k_count<true, false, true>, k_count<true, true>)
+                       : go(k_count<false, false>, k_count<false, false, true>,
+                            k_count<false, true>);
   });
 }
 
@@ -2000,8 +2013,8 @@ int vt_adjoint(const vt_cloud *cc, const double *d_start, const double *d_end, s
     };
     float ms = 0.0f;
     if (!d_counts) {
-      rc = c->periodic ? count(k_count<true, false>, k_count<true, true>)
-                       : count(k_count<false, false>, k_count<false, true>);
+      rc = c->periodic ? count(k_count<true, false, true>, k_count<true, true>)
+                       : count(k_count<false, false, true>, k_count<false, true>);
       if (rc) return rc;
       ms = g_stats.kernel_ms;
     }
