@@ -341,6 +341,7 @@ template <bool PER, int G, int kShare>
 __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 4 ? 3 : 4))) void k_march(
     DevCloud C, NbLists N, MarchRays R, MarchBufs B, double far, Stats *stats, int batch) {
   constexpr int kChunk = G * kShare;  // list entries a group takes at once
+  static_assert(kShare % 4 == 0 && kNbMax % kChunk == 0, "lists are read in whole chunks");
   constexpr int kRays = 64 / G;
   // Generators of a leaf whose loads are in flight together.
   constexpr int kSearchChunk = G == 4 ? 5 : 3;
@@ -383,19 +384,13 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 4 ? 3 :
   auto read_ids = [&](int pos) {
     const uint4 *p =
         reinterpret_cast<const uint4 *>(N.nb + (size_t)list * kNbMax + kChunk * pos + kShare * gl);
-    if constexpr (kShare == 2) {
-      const uint64_t q = gld(reinterpret_cast<const uint64_t *>(p));
-      id[0] = (uint32_t)q;
-      id[1] = (uint32_t)(q >> 32);
-    } else {
 #pragma unroll
-      for (int i = 0; i < kShare; i += 4) {
-        const uint4 q = gld(p + i / 4);
-        id[i] = q.x;
-        id[i + 1] = q.y;
-        id[i + 2] = q.z;
-        id[i + 3] = q.w;
-      }
+    for (int i = 0; i < kShare; i += 4) {
+      const uint4 q = gld(p + i / 4);
+      id[i] = q.x;
+      id[i + 1] = q.y;
+      id[i + 2] = q.z;
+      id[i + 3] = q.w;
     }
   };
   // The queue's parts, this block's own first.
@@ -1208,16 +1203,18 @@ static void march_batch_p(const MarchCall &m) {
   // Rays per wave.  The fewer rays there are, the more lanes are worth a ray:
   // its crossings are a chain, and the last rays' chains end the launch.
   // Measured with 4, 8 and 16 lanes (ms): 512^2 rays through clustered periodic
-  // cells 7.3, 8.4, 10.5; 384^2 4.8, 4.5, 5.6; 256^2 5.2, 4.1, 4.3; 16^2 .17,
-  // .17, .11; without images, where searches are cheaper, 300 x 257 rays 2.9,
-  // 3.2, 3.9; 128^2 .61, .59, .65.
+  // cells 7.1, 8.4, 10.5; 384^2 4.8, 4.2, 5.6; 256^2 4.9, 3.9, 4.1; 16^2 .17,
+  // .17, .10; without images, where searches are cheaper, 300 x 257 rays 2.8,
+  // 3.2, 3.9; 128^2 .61, .52, .65.  Chunks of 32 or 64 entries save rounds (16
+  // entries: 384^2 4.6, 300 x 257 3.0, 128^2 .57), but with images and 4 lanes
+  // they cost registers (512^2 7.8).
   const int64_t many = (PER ? 768ll : 256ll) * m.cus;
   if (m.R.n >= many)
-    go(k_march<PER, 4, 4>, 16, 4);  // (searches for 3, 6 or 8 waiting rays: no better)
+    go(k_march<PER, 4, PER ? 4 : 8>, 16, 4);  // (searches for 3, 6 or 8 waiting rays: no better)
   else if (m.R.n >= 64ll * m.cus)
-    go(k_march<PER, 8, 2>, 8, 2);
+    go(k_march<PER, 8, 4>, 8, 2);
   else
-    go(k_march<PER, 16, 2>, 4, 1);
+    go(k_march<PER, 16, 4>, 4, 1);
 }
 
 void march_batch(const MarchCall &m, bool periodic) {
