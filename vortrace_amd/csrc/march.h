@@ -57,11 +57,13 @@ struct MarchBufs {
   // Per slot: the entry to march from (kNone: not at all), then the number
   // of cells (0: left to the engine).
   uint32_t *c0;
-  uint32_t *ctr;  // kMarchCounters words: slots taken of each part of the queue
+  // kMarchCounters words: slots taken of each part of the queue, and the starts
+  // left to k_locate_far.
+  uint32_t *ctr;
   int cap;
 };
 
-constexpr int kMarchCounters = kParts;
+constexpr int kMarchCounters = kParts + 1;
 
 struct MarchCall {
   DevCloud C;
@@ -87,7 +89,7 @@ void march_batch(const MarchCall &m, bool periodic);
 // Checks the batch's envelopes and hands their segments to `io`'s sinks.
 template <class IO>
 void march_finish(const MarchCall &m, bool periodic, const IO &io);
-// The most workgroups k_locate runs (its scratch is sized by it).
+// The most workgroups k_locate_far runs (its scratch is sized by it).
 int march_locate_grid(int cus);
 
 // Records a ray's segments in one run of the pool (RecordIO for the march).

@@ -60,49 +60,6 @@ __device__ __forceinline__ int64_t xcd_block(int64_t b, int64_t nb) {
   return (b % kParts) * share + b / kParts;
 }
 
-// Every ray's start cell as entry 0 of its column, and 0 as the entry to march
-// from -- or kNone when the march cannot vouch for the start.  Also zeroes the
-// batch's queues.
-template <bool PER>
-__global__ __launch_bounds__(kBlock) void k_locate(DevCloud C, Scratch S, MarchRays R,
-                                                   MarchBufs B) {
-  const int tid = threadIdx.x;
-  const int gtid = blockIdx.x * kBlock + tid;
-  if (gtid < kMarchCounters) gst(B.ctr + gtid, 0u);
-  const LaneInfo li{tid, gtid, gtid >> 6, (int)(tid & 63)};
-  KStack st = make_stack(S, li);
-  for (int64_t j = gtid; j < R.n; j += (int64_t)gridDim.x * kBlock) {
-    const int64_t ray = march_ray(R, j);
-    RayGeom r;
-    make_ray(R.start + 3 * ray, R.end + 3 * ray, r);
-    uint32_t id[2];
-    double d[2];
-    query_reg<2, PER>(C, r.a[0], r.a[1], r.a[2], id, d, st);
-    double scale;
-    const double delta = clearance(C, r, scale);
-    const bool ok = id[0] != kNone && d[1] - d[0] > delta && r.len > 1e-6 && r.len < 1e30 &&
-                    scale < 1e15 && !st.overflow;
-    if (ok) {
-      const uint32_t c0 = id[0];
-      uint32_t code = kNbCentre;
-      if constexpr (PER) {
-        // The generator's image nearest to the start.
-        const double2 xy = gld(reinterpret_cast<const double2 *>(C.gen + c0));
-        const double g[3] = {xy.x, xy.y, gld(&C.gen[c0].z)};
-        int im[3];
-#pragma unroll
-        for (int k = 0; k < 3; ++k) {
-          const double e = r.a[k] - g[k];
-          im[k] = e > 0.5 * C.box[k] ? 1 : (e < -0.5 * C.box[k] ? -1 : 0);
-        }
-        code = image_code(im[0], im[1], im[2]);
-      }
-      gst(B.seq + (size_t)j * B.cap, make_uint4(0u, 0u, c0 | (code << kNbSlotBits), 0u));
-    }
-    gst(B.c0 + j, ok ? 0u : kNone);
-  }
-}
-
 // A value from another lane of a group of 4 or 16: lanes 1 or 2 apart, or
 // mirrored within 8 or 16 (after the steps before, each of those lanes holds
 // its own quad's or half's result).
@@ -111,6 +68,233 @@ __device__ __forceinline__ uint32_t group_swap(uint32_t v) {
   constexpr int ctrl = STEP == 0 ? 0xB1 : (STEP == 1 ? 0x4E : (STEP == 2 ? 0x141 : 0x140));
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
 }
+// The nearest generator so far.
+struct Near {
+  double d2 = INFINITY;
+  uint32_t name = kNone;
+  __device__ __forceinline__ void offer(double d, uint32_t id) {
+    name = d < d2 ? +id : +name;
+    d2 = fmin(d, d2);
+  }
+  template <int STEP>
+  __device__ __forceinline__ void swap_in() {
+    const uint64_t b = (uint64_t)__double_as_longlong(d2);
+    const uint32_t lo = group_swap<STEP>((uint32_t)b), hi = group_swap<STEP>((uint32_t)(b >> 32));
+    const uint32_t id = group_swap<STEP>(name);
+    offer(__longlong_as_double((long long)(((uint64_t)hi << 32) | lo)), id);
+  }
+  // The nearest of a group's lanes; equals: any of them, alike in every lane.
+  template <int G>
+  __device__ __forceinline__ void reduce() {
+    swap_in<0>();
+    swap_in<1>();
+    if constexpr (G > 8) {
+      swap_in<2>();
+      swap_in<3>();
+    }
+    name = __shfl(name, (threadIdx.x & 63) & ~(G - 1));
+  }
+};
+
+__device__ __forceinline__ void load_gen(const DevCloud &C, uint32_t slot, double (&g)[3]) {
+  const double2 xy = gld(reinterpret_cast<const double2 *>(C.gen + slot));
+  g[0] = xy.x;
+  g[1] = xy.y;
+  g[2] = gld(&C.gen[slot].z);
+}
+
+// Empties a batch's queues.
+__global__ __launch_bounds__(64) void k_zero(uint32_t *ctr) {
+  if (threadIdx.x < kMarchCounters) gst(ctr + threadIdx.x, 0u);
+}
+
+// Every ray's start cell as entry 0 of its column, and 0 as the entry to march
+// from -- or kNone when the march cannot vouch for the start.
+//
+// G lanes per ray: the tree is descended once, to the start's leaf; from the
+// nearest generator there the lists lead to the nearest of all (any nearer one
+// is within twice its distance, and a list that reaches that far has it).  Starts
+// whose lists do not reach that far are left to k_locate_far, in `rest`.  Bound
+// by the chain of reads, some ten of the descent and two per cell: with a search
+// of the tree per lane 256 rays took 212 us (its images and backtracking, lanes
+// apart) and 262,144 rays 720 us; now 11 us, and 118 + 234 us.
+template <bool PER, int G>
+__global__ __launch_bounds__(kBlock) void k_locate(DevCloud C, NbLists N, MarchRays R, MarchBufs B,
+                                                   uint32_t *rest) {
+  constexpr int kChunk = 4 * G;
+  const int tid = threadIdx.x;
+  const int gtid = blockIdx.x * kBlock + tid;
+  const int gl = tid & (G - 1), lead = (tid & 63) & ~(G - 1);
+  for (int64_t j = gtid / G; j < R.n; j += (int64_t)gridDim.x * (kBlock / G)) {
+    const int64_t ray = march_ray(R, j);
+    RayGeom r;
+    make_ray(R.start + 3 * ray, R.end + 3 * ray, r);
+    double scale;
+    const double delta = clearance(C, r, scale);
+    const bool sane = r.len > 1e-6 && r.len < 1e30 && scale < 1e15;
+    uint32_t c = kNone, code = kNbCentre;
+    bool sure = false;
+    if (sane) {
+      // The leaf of the start, folded into the box.
+      double q[3];
+#pragma unroll
+      for (int d = 0; d < 3; ++d) {
+        q[d] = r.a[d];
+        if constexpr (PER) {
+          const double off = q[d] - 0.5 * (C.rb_lo[d] + C.rb_hi[d]);
+          if (off > 0.5 * C.box[d]) q[d] -= C.box[d];
+          if (off < -0.5 * C.box[d]) q[d] += C.box[d];
+        }
+      }
+      uint32_t cur = C.rroot;
+      while (!(cur & kRefLeaf)) {
+        const DRecV rec = load_rec(C.recs, cur);
+        double cut;
+        cur = choose(rec.x, sel3(q[0], q[1], q[2], rec.x.dim), cut) ? rec.x.c1 : rec.x.c2;
+        if (!(cur & kRefLeaf)) {
+          const DNodeV nd = rec_child(rec, cur & 1u);
+          cur = choose(nd, sel3(q[0], q[1], q[2], nd.dim), cut) ? nd.c1 : nd.c2;
+        }
+      }
+      const uint32_t s0 = cur & kSlotMask, end = (uint32_t)gld(&C.gen[s0].end);
+      Near near;
+      for (uint32_t t = s0 + gl; t < end; t += G) {
+        double g[3], d2 = 0.0;
+        load_gen(C, t, g);
+#pragma unroll
+        for (int d = 0; d < 3; ++d) d2 = __builtin_fma(g[d] - q[d], g[d] - q[d], d2);
+        near.offer(d2, t);
+      }
+      near.template reduce<G>();
+      c = near.name;
+      double gb[3], w[3];
+      load_gen(C, c, gb);
+      if constexpr (PER) {
+        // The image nearest to the start.
+        int im[3];
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          const double e = r.a[d] - gb[d];
+          im[d] = e > 0.5 * C.box[d] ? 1 : (e < -0.5 * C.box[d] ? -1 : 0);
+        }
+        code = image_code(im[0], im[1], im[2]);
+      }
+      bool go = true;
+      for (int move = 0; go && move < 64; ++move) {
+        double v2 = 0.0;
+#pragma unroll
+        for (int d = 0; d < 3; ++d) {
+          w[d] = r.a[d] - gb[d];
+          if (PER && code != kNbCentre) w[d] -= image_axis(code, d) * C.box[d];
+          v2 = __builtin_fma(w[d], w[d], v2);
+        }
+        const double complete = gld(N.r2 + c);
+        near = Near();
+        go = false;
+        for (int pos = 0; pos < kNbMax / kChunk; ++pos) {
+          const uint4 ids =
+              gld(reinterpret_cast<const uint4 *>(N.nb + (size_t)c * kNbMax + pos * kChunk) + gl);
+          const uint32_t id[4] = {ids.x, ids.y, ids.z, ids.w};
+          double g[4][3];
+#pragma unroll
+          for (int i = 0; i < 4; ++i) load_gen(C, id[i] == kNone ? c : id[i] & kNbSlotMask, g[i]);
+          double last = 0.0;
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const uint32_t rel = id[i] >> kNbSlotBits;
+            bool named = true;
+            double dd = 0.0, d2 = 0.0;
+#pragma unroll
+            for (int d = 0; d < 3; ++d) {
+              double e = g[i][d] - gb[d];
+              if (PER && id[i] != kNone) {
+                if (rel != kNbCentre) e += image_axis(rel, d) * C.box[d];
+                named &= abs(image_axis(rel, d) + image_axis(code, d)) <= 1;
+              }
+              dd = __builtin_fma(e, e, dd);
+              d2 = __builtin_fma(e - w[d], e - w[d], d2);
+            }
+            if (id[i] != kNone) near.offer(d2, named ? id[i] : kNone);
+            last = id[i] == kNone ? (double)INFINITY : dd;
+          }
+          near.template reduce<G>();
+          last = __shfl(last, lead + G - 1);
+          if (near.d2 < v2) {
+            go = near.name != kNone;  // (an image the march cannot name: searched for)
+            break;
+          }
+          const bool ended = last == (double)INFINITY || pos + 1 == kNbMax / kChunk;
+          const double lim = ended ? complete : last * 0.999998;
+          const double gap = lim - delta;
+          if (gap > 0.0 && gap * gap > 4.000008 * lim * v2) {
+            sure = true;
+            break;
+          }
+          if (ended) break;
+        }
+        if (go) {
+          c = near.name & kNbSlotMask;
+          if constexpr (PER) code += (near.name >> kNbSlotBits) - kNbCentre;
+          load_gen(C, c, gb);
+        }
+        if (sure && !(near.d2 - v2 > delta)) c = kNone;  // a tie: the engine's
+      }
+    }
+    if (gl == 0) {
+      if (sane && !sure) {
+        gst(rest + atomicAdd(B.ctr + kParts, 1u), (uint32_t)j);
+      } else {
+        if (c != kNone)
+          gst(B.seq + (size_t)j * B.cap, make_uint4(0u, 0u, c | (code << kNbSlotBits), 0u));
+        gst(B.c0 + j, c != kNone ? 0u : kNone);
+      }
+    }
+  }
+}
+
+// The starts k_locate left: a search of the tree each.
+template <bool PER>
+__global__ __launch_bounds__(kBlock) void k_locate_far(DevCloud C, Scratch S, MarchRays R,
+                                                       MarchBufs B, const uint32_t *rest) {
+  const int tid = threadIdx.x;
+  const int gtid = blockIdx.x * kBlock + tid;
+  const LaneInfo li{tid, gtid, gtid >> 6, (int)(tid & 63)};
+  KStack st = make_stack(S, li);
+  const uint32_t n = gld(B.ctr + kParts);
+  // Spread over the waves, as a wave's searches take different ways (262,144
+  // rays through clumps: 234 us, with full waves 700 us).
+  const uint32_t waves = gridDim.x * (kBlock / 64);
+  for (uint32_t i = (tid & 63) * waves + (gtid >> 6); i < n; i += 64 * waves) {
+    const uint32_t j = gld(rest + i);
+    const int64_t ray = march_ray(R, j);
+    RayGeom r;
+    make_ray(R.start + 3 * ray, R.end + 3 * ray, r);
+    double scale;
+    const double delta = clearance(C, r, scale);
+    uint32_t id[2];
+    double d[2];
+    query_reg<2, PER>(C, r.a[0], r.a[1], r.a[2], id, d, st);
+    const bool ok = id[0] != kNone && d[1] - d[0] > delta && !st.overflow;
+    if (ok) {
+      uint32_t code = kNbCentre;
+      if constexpr (PER) {
+        // The generator's image nearest to the start.
+        double g[3];
+        load_gen(C, id[0], g);
+        int im[3];
+#pragma unroll
+        for (int k = 0; k < 3; ++k) {
+          const double e = r.a[k] - g[k];
+          im[k] = e > 0.5 * C.box[k] ? 1 : (e < -0.5 * C.box[k] ? -1 : 0);
+        }
+        code = image_code(im[0], im[1], im[2]);
+      }
+      gst(B.seq + (size_t)j * B.cap, make_uint4(0u, 0u, id[0] | (code << kNbSlotBits), 0u));
+    }
+    gst(B.c0 + j, ok ? 0u : kNone);
+  }
+}
+
 // The three nearest candidates' places (where they come within the clearance;
 // floats, good to kKeyTol), and the names of the nearer two.  Floats order all
 // but a millionth of the exits; the rest, and every exit taken, are computed
@@ -1190,8 +1374,21 @@ int march_locate_grid(int cus) { return 4 * cus; }
 
 template <bool PER>
 static void march_batch_p(const MarchCall &m) {
-  const int grid = (int)std::min<int64_t>(march_locate_grid(m.cus), (m.R.n + kBlock - 1) / kBlock);
-  k_locate<PER><<<grid, kBlock, 0, m.st>>>(m.C, m.S, m.R, m.B);
+  k_zero<<<1, 64, 0, m.st>>>(m.B.ctr);
+  // (The batch's own part of the list of rays left to the engine, empty yet.)
+  uint32_t *rest = m.fall + m.R.base;
+  auto locate = [&](auto kernel, int lanes) {
+    const int64_t blocks = (m.R.n * lanes + kBlock - 1) / kBlock;
+    kernel<<<(int)std::min<int64_t>(32ll * m.cus, blocks), kBlock, 0, m.st>>>(m.C, m.N, m.R, m.B,
+                                                                             rest);
+  };
+  if (m.R.n >= 64ll * m.cus)
+    locate(k_locate<PER, 4>, 4);
+  else
+    locate(k_locate<PER, 16>, 16);
+  const int64_t far_blocks = (m.R.n + 1) / 2;
+  k_locate_far<PER><<<(int)std::min<int64_t>(march_locate_grid(m.cus), far_blocks), kBlock, 0,
+                      m.st>>>(m.C, m.S, m.R, m.B, rest);
   // As many waves as the chip holds at once, or as the rays need.
   double far = DBL_MAX;
   if (PER) far = 0.2 * std::min(m.C.box[0], std::min(m.C.box[1], m.C.box[2]));
