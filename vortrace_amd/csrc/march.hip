@@ -993,11 +993,10 @@ __global__ __launch_bounds__(64) __attribute__((amdgpu_waves_per_eu(G == 4 ? 3 :
   if (lane == 0 && nball) atomicAdd(&stats->queries, (unsigned long long)nball);
 }
 
-// Rays per wave of the replay, cells whose entries it holds in LDS (at least
-// the longest ray's), and intervals it can hold for its lanes.
+// Rays per wave of the replay, and cells whose entries it holds in LDS (at least
+// the longest ray's).
 constexpr int kReplayRays = 4;
 constexpr int kReplayCells = 576;
-constexpr int kPool = 512;
 
 // The replay of the recursion (see march.h) over the lanes of a wave.  An item
 // is an interval (i, j), j >= i + 2, of a ray's cells that the recursion visits
@@ -1014,7 +1013,7 @@ __global__ __launch_bounds__(64) void k_replay(DevCloud C, MarchRays R, MarchBuf
   extern __shared__ uint4 dyn[];  // room entries, then where the recursion inserts them
   uint4 *ent = dyn;
   double *ins = reinterpret_cast<double *>(dyn + room);
-  __shared__ uint64_t item[kPool];
+  uint64_t *item = reinterpret_cast<uint64_t *>(ins + (PER ? room : 0));  // the pool
   __shared__ double geo[7][kReplayRays];
   __shared__ int cells[kReplayRays], start[kReplayRays];
   __shared__ uint32_t bad[kReplayRays];
@@ -1427,8 +1426,13 @@ void march_finish(const MarchCall &m, bool periodic, const IO &io) {
     return (unsigned)(((m.R.n + rays - 1) / rays + kParts - 1) / kParts * kParts);
   };
   const int room = std::max(kReplayCells, m.B.cap);
-  const size_t lds = (size_t)room * (sizeof(uint4) + (periodic ? sizeof(double) : 0));
-  const int pool = std::min(m.pool, kPool);
+  // Intervals a wave holds: breadth grows by a wave's worth per level below the
+  // 64th interval, so rays of up to 640 cells need 256 (an overflow leaves the
+  // ray to the engine).  512 for all took a wave per CU: 2M cells, 512^2 rays
+  // .96 ms against .88, 4M cells 3.07 against 2.78.
+  const int pool = std::min(m.pool, m.B.cap <= 640 ? 256 : 512);
+  const size_t lds = (size_t)room * (sizeof(uint4) + (periodic ? sizeof(double) : 0)) +
+                     (size_t)pool * sizeof(uint64_t);
   if (periodic)
     k_replay<true><<<waves(kReplayRays), 64, lds, m.st>>>(m.C, m.R, m.B, room, pool, m.fall,
                                                           m.stats);
