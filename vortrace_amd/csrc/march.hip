@@ -1343,8 +1343,13 @@ __global__ __launch_bounds__(64) void k_emit(MarchRays R, MarchBufs B, IO io, Er
         const uint4 e = gld(src + k);
         const double b = k + 1 < n ? at(gld(src + k + 1)) : end;
         SegRec *o = io.pool.rec + base + off + k;
-        gst_nt(reinterpret_cast<uint4 *>(o), make_uint4(e.z & kNbSlotMask, id, (uint32_t)k, 0u));
-        gst_nt(&o->ds, b - at(e));
+        // Both halves whole, through the cache, which joins them: 1.51 ms for
+        // 52M segments of 8M cells, against 2.22 with the padding left out and
+        // streaming stores.
+        const uint64_t ds = (uint64_t)__double_as_longlong(b - at(e));
+        gst(reinterpret_cast<uint4 *>(o), make_uint4(e.z & kNbSlotMask, id, (uint32_t)k, 0u));
+        gst(reinterpret_cast<uint4 *>(o) + 1,
+            make_uint4((uint32_t)ds, (uint32_t)(ds >> 32), 0u, 0u));
       }
     }
   }
