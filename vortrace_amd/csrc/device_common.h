@@ -73,6 +73,12 @@ struct Stats {
   unsigned long long fallback;         // march: rays left to the engine
 };
 
+// What a call brings back.
+struct CallRec {
+  ErrRec err;
+  Stats stats;
+};
+
 // The ray engine splits its rays into kParts contiguous partitions, one per
 // XCD: workgroups are dispatched to the XCDs round-robin, so workgroup b runs
 // on XCD b mod 8 and its lanes take rays from partition b mod 8 first.  Rays

@@ -103,13 +103,9 @@ __device__ __forceinline__ void load_gen(const DevCloud &C, uint32_t slot, doubl
   g[2] = gld(&C.gen[slot].z);
 }
 
-// Empties a batch's queues.
-__global__ __launch_bounds__(64) void k_zero(uint32_t *ctr) {
-  if (threadIdx.x < kMarchCounters) gst(ctr + threadIdx.x, 0u);
-}
-
 // Every ray's start cell as entry 0 of its column, and 0 as the entry to march
-// from -- or kNone when the march cannot vouch for the start.
+// from -- or kNone when the march cannot vouch for the start.  Also empties the
+// batch's queues.
 //
 // G lanes per ray: the tree is descended once, to the start's leaf; from the
 // nearest generator there the lists lead to the nearest of all (any nearer one
@@ -125,6 +121,7 @@ __global__ __launch_bounds__(kBlock) void k_locate(DevCloud C, NbLists N, MarchR
   const int tid = threadIdx.x;
   const int gtid = blockIdx.x * kBlock + tid;
   const int gl = tid & (G - 1), lead = (tid & 63) & ~(G - 1);
+  if (gtid < kParts) gst(B.ctr + gtid, 0u);
   for (int64_t j = gtid / G; j < R.n; j += (int64_t)gridDim.x * (kBlock / G)) {
     const int64_t ray = march_ray(R, j);
     RayGeom r;
@@ -1018,6 +1015,7 @@ __global__ __launch_bounds__(64) void k_replay(DevCloud C, MarchRays R, MarchBuf
   __shared__ int cells[kReplayRays], start[kReplayRays];
   __shared__ uint32_t bad[kReplayRays];
   const int lane = threadIdx.x;
+  if (blockIdx.x == 0 && lane == 0) gst(B.ctr + kParts, 0u);  // for the next batch's starts
   const int64_t j0 = xcd_block(blockIdx.x, gridDim.x) * kReplayRays;
   const int64_t j = j0 + lane;
   const bool mine = lane < kReplayRays && j < R.n;
@@ -1378,7 +1376,6 @@ int march_locate_grid(int cus) { return 4 * cus; }
 
 template <bool PER>
 static void march_batch_p(const MarchCall &m) {
-  k_zero<<<1, 64, 0, m.st>>>(m.B.ctr);
   // (The batch's own part of the list of rays left to the engine, empty yet.)
   uint32_t *rest = m.fall + m.R.base;
   auto locate = [&](auto kernel, int lanes) {

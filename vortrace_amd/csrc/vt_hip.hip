@@ -345,7 +345,8 @@ struct vt_cloud {
   Gen *d_gen = nullptr;
   double *d_fields = nullptr;
   uint32_t *d_slot_id = nullptr;
-  ErrRec *d_err = nullptr;
+  CallRec *d_call = nullptr;    // a call's error record and statistics,
+  ErrRec *d_err = nullptr;      // and its two parts
   Stats *d_stats = nullptr;
   Scratch scratch{};
   size_t scratch_lanes = 0;
@@ -373,7 +374,7 @@ struct vt_cloud {
 
   void free_device() {
     for (void *p : {(void *)d_nodes, (void *)d_recs, (void *)d_gen, (void *)d_fields, (void *)d_slot_id,
-                    (void *)d_err, (void *)d_stats, (void *)scratch.knn_spill,
+                    (void *)d_call, (void *)scratch.knn_spill,
                     (void *)scratch.walk_tag, (void *)scratch.walk_s,
                     (void *)scratch.big_id, (void *)scratch.big_d, (void *)help_ev,
                     (void *)help_steal, (void *)d_defer, (void *)d_nb, (void *)d_nr2,
@@ -403,6 +404,7 @@ struct vt_cloud {
     d_gen = nullptr;
     d_fields = nullptr;
     d_slot_id = nullptr;
+    d_call = nullptr;
     d_err = nullptr;
     d_stats = nullptr;
     scratch = Scratch{};
@@ -528,9 +530,26 @@ void ensure_defer(vt_cloud *c, size_t nrays) {
   c->defer_cap = nrays;
 }
 
+// Zeroes a call's error record and statistics (a kernel, so the call issues
+// no memset).
+__global__ void k_clear_call(ErrRec *err, Stats *stats) {
+  uint32_t *e = reinterpret_cast<uint32_t *>(err);
+  uint32_t *s = reinterpret_cast<uint32_t *>(stats);
+  constexpr int ne = sizeof(ErrRec) / 4, ns = sizeof(Stats) / 4;
+  static_assert(sizeof(ErrRec) % 4 == 0 && sizeof(Stats) % 4 == 0, "word-sized records");
+  for (int i = threadIdx.x; i < ne + ns; i += blockDim.x) {
+    if (i < ne)
+      e[i] = 0u;
+    else
+      s[i - ne] = 0u;
+  }
+}
+
+// One launch and one copy back a call: with two fills and two copies they were
+// a third of a 16^2 call.
 void reset_call(vt_cloud *c, hipStream_t st) {
-  HIP_OK(hipMemsetAsync(c->d_err, 0, sizeof(ErrRec), st));
-  HIP_OK(hipMemsetAsync(c->d_stats, 0, sizeof(Stats), st));
+  k_clear_call<<<1, 64, 0, st>>>(c->d_err, c->d_stats);
+  HIP_OK(hipGetLastError());
 }
 
 // Waits for the call, copies the error record and statistics back and turns
@@ -539,11 +558,11 @@ void reset_call(vt_cloud *c, hipStream_t st) {
 // `fallback` receives the rays a march left to the engine.
 int finish_call(vt_cloud *c, hipStream_t st, hipEvent_t e0, hipEvent_t e1, bool more = false,
                 int64_t *fallback = nullptr) {
-  ErrRec er;
-  Stats ss;
-  HIP_OK(hipMemcpyAsync(&er, c->d_err, sizeof er, hipMemcpyDeviceToHost, st));
-  HIP_OK(hipMemcpyAsync(&ss, c->d_stats, sizeof ss, hipMemcpyDeviceToHost, st));
+  CallRec call;
+  HIP_OK(hipMemcpyAsync(&call, c->d_call, sizeof call, hipMemcpyDeviceToHost, st));
   HIP_OK(hipStreamSynchronize(st));
+  const ErrRec &er = call.err;
+  const Stats &ss = call.stats;
   float ms = 0;
   if (e0 && e1) HIP_OK(hipEventElapsedTime(&ms, e0, e1));
   if (!more) g_stats = vt_call_stats{};
@@ -722,7 +741,7 @@ bool march_pays(const vt_cloud *c) { return c->d_nb != nullptr && help_events() 
 // The march's work buffers for at most `n` rays, in batches of what fits in
 // kMarchBytes.  Returns the batch size.
 constexpr size_t kMarchBytes = (size_t)9 << 29;  // 4.5 GiB
-int64_t ensure_march(vt_cloud *c, int64_t n) {
+int64_t ensure_march(vt_cloud *c, int64_t n, hipStream_t st) {
   // Cells a ray may cross: several times the mean of a uniform mesh along a
   // box diagonal; longer rays run in the engine.
   int cap = (int)(2.6 * std::cbrt((double)c->n)) + 64;
@@ -740,6 +759,7 @@ int64_t ensure_march(vt_cloud *c, int64_t n) {
     c->march.seq = dev_alloc<uint4>((size_t)cap * rays);
     c->march.c0 = dev_alloc<uint32_t>((size_t)rays);
     c->march.ctr = dev_alloc<uint32_t>(kMarchCounters);
+    HIP_OK(hipMemsetAsync(c->march.ctr, 0, kMarchCounters * sizeof(uint32_t), st));
     c->march_rays = (size_t)rays;
   }
   if (c->fall_cap < (size_t)n) {
@@ -761,7 +781,7 @@ int march(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io
   MarchCall m{};
   m.cus = num_cus(c->device);
   ensure_scratch(c, (size_t)march_locate_grid(m.cus) * kBlock);
-  const int64_t rays = ensure_march(c, n);
+  const int64_t rays = ensure_march(c, n, st);
   m.C = c->dc;
   m.S = c->scratch;
   m.N = NbLists{c->d_nb, c->d_nr2, c->d_boxes};
@@ -1111,21 +1131,6 @@ constexpr size_t kNoAllocBytes = size_t(128) << 20;  // 128 MiB per device
 constexpr int64_t kNoAllocMaxRays = int64_t(1) << 22;  // deferred list: 16 MiB at most
 __device__ __align__(256) unsigned char scratch[kNoAllocBytes];
 
-// Zeroes a call's error record and statistics (a kernel, so the call issues
-// no memset).
-__global__ void k_clear_call(ErrRec *err, Stats *stats) {
-  uint32_t *e = reinterpret_cast<uint32_t *>(err);
-  uint32_t *s = reinterpret_cast<uint32_t *>(stats);
-  constexpr int ne = sizeof(ErrRec) / 4, ns = sizeof(Stats) / 4;
-  static_assert(sizeof(ErrRec) % 4 == 0 && sizeof(Stats) % 4 == 0, "word-sized records");
-  for (int i = threadIdx.x; i < ne + ns; i += blockDim.x) {
-    if (i < ne)
-      e[i] = 0u;
-    else
-      s[i - ne] = 0u;
-  }
-}
-
 }  // namespace vt
 
 namespace {
@@ -1408,8 +1413,9 @@ int vt_cloud_upload(vt_cloud *c) {
     c->d_gen = dev_alloc<Gen>(c->n + kLeafMaxSize);
     c->d_fields = dev_alloc<double>(fslot.size());
     c->d_slot_id = dev_alloc<uint32_t>(c->n);
-    c->d_err = dev_alloc<ErrRec>(1);
-    c->d_stats = dev_alloc<Stats>(1);
+    c->d_call = dev_alloc<CallRec>(1);
+    c->d_err = &c->d_call->err;
+    c->d_stats = &c->d_call->stats;
     if (!dt.nodes.empty())
       HIP_OK(hipMemcpy(c->d_nodes, dt.nodes.data(), dt.nodes.size() * sizeof(DNode),
                        hipMemcpyHostToDevice));
