@@ -511,8 +511,8 @@ __device__ __forceinline__ float box_below2(const float (&lo)[3], const float (&
 //
 // Bound by VALU issue (64 % of the cycles) and, with three waves per SIMD, by the
 // latency of the chain list -> generators -> exit -> next list.  2M clustered
-// cells, 512^2 rays (126 crossings each): 7.4 ms, of which the 1.1 % of
-// crossings that search take a quarter; 1M such cells, 1024^2 rays: 2 x 10.3 ms.
+// cells, 512^2 rays (126 crossings each): 7.1 ms, of which the 1.1 % of
+// crossings that search take a quarter; 1M such cells, 1024^2 rays: 2 x 10.1 ms.
 // With FP64 keys, the image shifts computed at each use and all of the ray in
 // registers it was 8.0 and 2 x 11.5 ms; the keys in scratch memory (see merge)
 // cost 1.2 ms, two waves per SIMD 1.4 ms, and four, which spill here, nothing

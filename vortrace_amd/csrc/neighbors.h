@@ -7,8 +7,9 @@
 // the leaf in slot order, every generator within that radius of the leaf's box
 // is collected from the kd-tree (64 nodes tested at a time), and each
 // generator of the leaf ranks the collected ones by distance.  A leaf's
-// generators share one traversal and one set of candidates.  2M clustered
-// points: 14 ms.  64 entries: at 48, 2 % of the crossings of a clustered mesh
+// generators share one traversal and one set of candidates.  Bound by VALU
+// issue, the ranking a third of it: 2M clustered points 12.1 ms, 8M 29.0 (13.9
+// and 39.7 with ties ranked in the same pass).  64 entries: at 48, 2 % of the crossings of a clustered mesh
 // have more generators in reach than the list holds, at 64 1.2 %, at 96 0.9 %.
 #pragma once
 #include "knn.h"
@@ -26,7 +27,7 @@ struct NbShared {
   uint32_t stack[kNbStack];
   uint32_t leaves[kNbLeaves];
   uint32_t cand[kNbCand];
-  float key[kNbSort];
+  alignas(16) float key[kNbSort];
   uint32_t ent[kNbSort];
 };
 
@@ -298,15 +299,27 @@ __global__ __launch_bounds__(64) void k_neighbors(DevCloud C, uint32_t *nb, floa
           n += __popcll(mk);
         }
       }
+      if (lane < 4 && n + lane < kNbSort) sh.key[n + lane] = INFINITY;
       __syncthreads();
-      // Rank by (distance, place); each lane places up to two candidates.
+      // Rank by (distance, place); each lane places up to two candidates.  The
+      // places are only looked at when two distances are equal (the ranks then
+      // do not add up to 0 + 1 + ... + n - 1).
       float k0 = lane < n ? sh.key[lane] : INFINITY;
       float k1 = lane + 64 < n ? sh.key[lane + 64] : INFINITY;
       int r0 = 0, r1 = 0;
-      for (int j = 0; j < n; ++j) {
-        const float kj = sh.key[j];
-        r0 += (kj < k0 || (kj == k0 && j < lane)) ? 1 : 0;
-        r1 += (kj < k1 || (kj == k1 && j < lane + 64)) ? 1 : 0;
+      for (int j = 0; j < n; j += 4) {
+        const float4 k = *reinterpret_cast<const float4 *>(sh.key + j);
+        r0 += (k.x < k0) + (k.y < k0) + (k.z < k0) + (k.w < k0);
+        r1 += (k.x < k1) + (k.y < k1) + (k.z < k1) + (k.w < k1);
+      }
+      int sum = (lane < n ? r0 : 0) + (lane + 64 < n ? r1 : 0);
+      for (int o = 32; o; o >>= 1) sum += __shfl_xor(sum, o);
+      if (sum != n * (n - 1) / 2) {
+        for (int j = 0; j < n; ++j) {
+          const float kj = sh.key[j];
+          r0 += (kj == k0 && j < lane) ? 1 : 0;
+          r1 += (kj == k1 && j < lane + 64) ? 1 : 0;
+        }
       }
       uint32_t *out = nb + (size_t)self * kNbMax;
       if (lane < n && r0 < kNbMax) gst(out + r0, sh.ent[lane]);

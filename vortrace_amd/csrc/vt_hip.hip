@@ -734,7 +734,7 @@ void launch(vt_cloud *c, K kernel, int64_t n, hipStream_t st, Timer &tm, A... ar
 
 // Whether a call's rays are marched first (march.h): whenever the cloud has
 // lists.  Measured at 2M clustered cells, 512^2 rays: 41.0 ms in the engine,
-// 11.7 ms marched; one ray across 20k cells 1.2 against 0.2 ms.
+// 9.8 ms marched; one ray across 20k cells 1.2 against 0.2 ms.
 // help_events = 0 asks for the engine alone.
 bool march_pays(const vt_cloud *c) { return c->d_nb != nullptr && help_events() > 0; }
 
