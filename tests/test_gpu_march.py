@@ -118,6 +118,17 @@ def test_lanes_per_ray(tuning, periodic, rays):
     np.testing.assert_array_equal(got[0], got[1])
 
 
+@pytest.mark.parametrize("rays,outside", [(64, 0), (64, 32), (64, 33), (3072, 3072),
+                                          (3073, 3073)])
+def test_few_rays_that_leave_the_box(tuning, rays, outside):
+    """Both sides of the choice between engine and march for a few rays."""
+    pos, rho = synthetic.uniform_mesh(100_000, seed=61)
+    pc = vt.ProjectionCloud(pos, rho, boundbox=[0.0, 100.0] * 3, periodic=False)
+    s, e = _chords(rays, 9, 1.0, 99.0)
+    s[:outside, 2] = -20.0
+    _compare(pc, s, e, f"{outside} of {rays} rays leave the box")
+
+
 @pytest.mark.parametrize("periodic", [False, True])
 def test_clump_beside_void(tuning, periodic):
     """Lists full of a clump's generators do not reach across the void."""

@@ -818,12 +818,47 @@ int march(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io
 // A call's rays: marched, and those the march leaves run in the engine
 // (fast(timer, list, n) and slow(timer, n) as in two_pass); or all of them in
 // the engine.
+// Rays that start or end farther than `edge` outside the generators' box.
+__global__ void k_leaving(DevCloud C, const double *s, const double *e, int64_t n, double edge,
+                          Stats *stats) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  bool out = false;
+  for (int d = 0; i < n && d < 3; ++d) {
+    const double a = gld(s + 3 * i + d), b = gld(e + 3 * i + d);
+    out |= fmin(a, b) < C.rb_lo[d] - edge || fmax(a, b) > C.rb_hi[d] + edge;
+  }
+  const uint64_t m = __ballot(out);
+  if ((threadIdx.x & 63) == 0 && m) atomicAdd(&stats->fallback, (unsigned long long)__popcll(m));
+}
+
+// Whether the engine projects these rays sooner than the march.  A march is a
+// chain of crossings, and outside the points of an open box each of them
+// searches the tree; the engine spreads a ray's intervals over a wave.  With
+// too few rays to fill the card that decides: 961 rays of a rotated view
+// through 740k uniform cells 1.2 ms in the engine, 2.0 marched; 4,096 rays 2.0
+// and 1.9; 961 through 20k cells .7 and .6; rays that stay inside .6 marched.
+bool engine_sooner(vt_cloud *c, const double *s, const double *e, int64_t n, hipStream_t st) {
+  if (c->periodic || c->n < 100000 || n > 12ll * num_cus(c->device)) return false;
+  double v = 1.0;
+  for (int d = 0; d < 3; ++d) v *= c->dc.rb_hi[d] - c->dc.rb_lo[d];
+  reset_call(c, st);
+  k_leaving<<<(int)((n + 255) / 256), 256, 0, st>>>(c->dc, s, e, n,
+                                                    2.0 * std::cbrt(v / (double)c->n), c->d_stats);
+  HIP_OK(hipGetLastError());
+  unsigned long long out = 0;
+  HIP_OK(hipMemcpyAsync(&out, &c->d_stats->fallback, sizeof out, hipMemcpyDeviceToHost, st));
+  HIP_OK(hipStreamSynchronize(st));
+  return 2 * (int64_t)out > n;
+}
+
 template <class IO, class Fast, class Slow>
 int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io,
-               hipStream_t st, Fast &&fast, Slow &&slow) {
+               hipStream_t st, Fast &&fast, Slow &&slow, bool projects = false) {
   const uint32_t *list = nullptr;
   int64_t left = n;
-  const bool marched = march_pays(c);
+  // (The kernels that count and list segments are slower than the march for any
+  // number of rays.)
+  const bool marched = march_pays(c) && !(projects && engine_sooner(c, s, e, n, st));
   if (marched) {
     const int rc = march(c, s, e, n, io, st, &left);
     if (rc || left == 0) return rc;
@@ -870,7 +905,8 @@ int project_p(vt_cloud *c, const double *s, const double *e, int64_t n, double *
       [&](Timer &tm, int64_t nd) {
         launch(c, k_project_x<MODE, PER, REC>, nd, st, tm, s, e, nd,
                (const uint32_t *)c->d_defer, out, nout, counts, pool, c->d_err, c->d_stats);
-      });
+      },
+      true);
 }
 
 template <int MODE, int NF, bool REC = false>
