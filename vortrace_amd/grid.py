@@ -149,10 +149,13 @@ def device_view(extent: ArrayLike, nres, bounds: ArrayLike,
         if not np.array_equal(rotation_matrix(yaw, pitch, roll), np.eye(3)):
             return None
         c = np.asarray(center)
-        if c.shape != (3,) or c.dtype.kind not in "iuf" or not np.all(np.isfinite(c)):
+        # (A long double centre is subtracted before it is rounded.)
+        if c.shape != (3,) or c.dtype.kind not in "iuf" or c.dtype.itemsize > 8 \
+                or not np.all(np.isfinite(c)):
             return None
     ext = np.asarray(extent)
-    if ext.shape not in ((2,), (2, 2)) or (ext.dtype != np.float64 and ext.dtype.kind not in "iu"):
+    # Narrow and unsigned integers wrap and divide in types of their own.
+    if ext.shape not in ((2,), (2, 2)) or ext.dtype not in (np.float64, np.int64):
         return None
     if not np.all(np.abs(ext.astype(np.float64)) < 2.0 ** 52):
         return None
