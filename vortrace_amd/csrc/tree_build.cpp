@@ -14,7 +14,9 @@
 #include "tree_build.h"
 
 #include <algorithm>
+#include <cmath>
 #include <cstring>
+#include <limits>
 #include <stdexcept>
 #include <string>
 #include <thread>
@@ -428,6 +430,42 @@ void load_tree_bytes(const uint8_t *b, size_t size, size_t npart, HostTree &out)
     t.nodes[nd.a].pb = nd.hi;
   }
   out = std::move(t);
+}
+
+bool tree_bounds_points(const HostTree &t, const double *pts) {
+  struct Box {
+    double lo[3], hi[3];
+  };
+  // Children follow their parent in pre-order, so backwards every child is
+  // done before its parent.
+  std::vector<Box> box(t.nodes.size());
+  for (size_t i = t.nodes.size(); i-- > 0;) {
+    const Node &nd = t.nodes[i];
+    Box &b = box[i];
+    if (nd.b & kLeafBit) {
+      for (int d = 0; d < 3; ++d) {
+        b.lo[d] = std::numeric_limits<double>::infinity();
+        b.hi[d] = -b.lo[d];
+      }
+      for (uint32_t s = nd.a; s < (nd.b & ~kLeafBit); ++s)
+        for (int d = 0; d < 3; ++d) {
+          const double x = pts[3 * (size_t)t.vind[s] + d];
+          if (!std::isfinite(x)) return false;
+          b.lo[d] = std::min(b.lo[d], x);
+          b.hi[d] = std::max(b.hi[d], x);
+        }
+      continue;
+    }
+    const Box &b1 = box[i + 1], &b2 = box[nd.a];
+    if (!(b1.hi[nd.b] <= nd.lo && nd.hi <= b2.lo[nd.b])) return false;
+    for (int d = 0; d < 3; ++d) {
+      b.lo[d] = std::min(b1.lo[d], b2.lo[d]);
+      b.hi[d] = std::max(b1.hi[d], b2.hi[d]);
+    }
+  }
+  for (int d = 0; d < 3; ++d)
+    if (!(t.bbox[d][0] <= box[0].lo[d] && box[0].hi[d] <= t.bbox[d][1])) return false;
+  return true;
 }
 
 }  // namespace vt

@@ -44,4 +44,9 @@ void make_device_tree(const HostTree &t, DeviceTree &out);
 void save_tree_bytes(const HostTree &t, std::vector<uint8_t> &out);
 void load_tree_bytes(const uint8_t *b, size_t size, size_t npart, HostTree &out);
 
+// Whether every cut and the root's box bound the points under them, as they do
+// in a tree built over these points.  A loaded dump need not (the points may
+// have moved since), nor a tree over NaN coordinates.
+bool tree_bounds_points(const HostTree &t, const double *pts);
+
 }  // namespace vt

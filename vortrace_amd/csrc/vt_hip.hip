@@ -335,6 +335,8 @@ struct vt_cloud {
   int periodic = 0, valid_rgba = 0;
   bool tree_built = false;  // host tree built and uploaded
   bool host_tree = false;   // host tree built
+  bool finite = true;       // every coordinate is
+  bool bounded = true;      // the tree's cuts bound the points under them
   HostTree tree;
   double build_seconds = 0;
 
@@ -1350,6 +1352,7 @@ int vt_cloud_create(const double *pos, size_t npart, const double *fields, size_
           c->pts.insert(c->pts.end(), p, p + 3);
           c->fields.insert(c->fields.end(), fields + i * nfields, fields + (i + 1) * nfields);
           c->orig_ids.push_back((int64_t)i);
+          c->finite &= std::isfinite(p[0]) && std::isfinite(p[1]) && std::isfinite(p[2]);
         }
       }
     } else {
@@ -1365,6 +1368,7 @@ int vt_cloud_create(const double *pos, size_t npart, const double *fields, size_
       for (size_t i = 0; i < npart; i++) {
         c->orig_ids[i] = (int64_t)i;
         for (int d = 0; d < 3; d++) {
+          c->finite &= (bool)std::isfinite(pos[3 * i + d]);
           pmin[d] = std::min(pmin[d], pos[3 * i + d]);
           pmax[d] = std::max(pmax[d], pos[3 * i + d]);
         }
@@ -1416,6 +1420,7 @@ int vt_cloud_build_host_tree(vt_cloud *c) {
     c->free_device();
     c->tree_built = false;
     c->host_tree = true;
+    c->bounded = c->finite;
     c->tree = std::move(t);
     if (g_verbose.load())
       std::printf("Tree build took %lld milliseconds.\n", (long long)(c->build_seconds * 1e3));
@@ -1484,8 +1489,9 @@ int vt_cloud_upload(vt_cloud *c) {
     d.root = dt.root;
     d.rroot = dt.rroot;
     // Neighbour lists for the march; without room for them every ray runs in
-    // the engine.
-    if (c->n <= kNbMaxPoints) {
+    // the engine.  So it does through a tree that does not bound its points:
+    // searches then find what the cuts let them, which only the engine repeats.
+    if (c->n <= kNbMaxPoints && c->bounded) {
       const size_t nn = dt.nodes.size();
       void *nb = nullptr, *nr = nullptr, *bx = nullptr;
       if (hipMalloc(&nb, c->n * kNbMax * sizeof(uint32_t)) == hipSuccess &&
@@ -1838,6 +1844,7 @@ int vt_cloud_load_tree(vt_cloud *c, const uint8_t *buf, size_t size, int upload)
     c->host_tree = true;
     c->build_seconds = 0.0;
     c->tree = std::move(t);
+    c->bounded = c->finite && tree_bounds_points(c->tree, c->pts.data());
     return upload ? vt_cloud_upload(c) : VT_OK;
   });
 }
