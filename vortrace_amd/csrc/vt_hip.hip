@@ -532,9 +532,10 @@ void ensure_defer(vt_cloud *c, size_t nrays) {
   c->defer_cap = nrays;
 }
 
-// Zeroes a call's error record and statistics (a kernel, so the call issues
-// no memset).
-__global__ void k_clear_call(ErrRec *err, Stats *stats) {
+// Zeroes a call's error record and statistics, and the length of the march's
+// list of starts when there is one (a kernel, so the call issues no memset).
+__global__ void k_clear_call(ErrRec *err, Stats *stats, uint32_t *starts) {
+  if (starts && threadIdx.x == 0) *starts = 0u;
   uint32_t *e = reinterpret_cast<uint32_t *>(err);
   uint32_t *s = reinterpret_cast<uint32_t *>(stats);
   constexpr int ne = sizeof(ErrRec) / 4, ns = sizeof(Stats) / 4;
@@ -548,9 +549,11 @@ __global__ void k_clear_call(ErrRec *err, Stats *stats) {
 }
 
 // One launch and one copy back a call: with two fills and two copies they were
-// a third of a 16^2 call.
+// a third of a 16^2 call.  Nothing a call counts in is left to an earlier one,
+// which may have failed between its launches or never run (stream capture).
 void reset_call(vt_cloud *c, hipStream_t st) {
-  k_clear_call<<<1, 64, 0, st>>>(c->d_err, c->d_stats);
+  k_clear_call<<<1, 64, 0, st>>>(c->d_err, c->d_stats,
+                                 c->march.ctr ? c->march.ctr + kParts : nullptr);
   HIP_OK(hipGetLastError());
 }
 
@@ -743,7 +746,7 @@ bool march_pays(const vt_cloud *c) { return c->d_nb != nullptr && help_events() 
 // The march's work buffers for at most `n` rays, in batches of what fits in
 // kMarchBytes.  Returns the batch size.
 constexpr size_t kMarchBytes = (size_t)9 << 29;  // 4.5 GiB
-int64_t ensure_march(vt_cloud *c, int64_t n, hipStream_t st) {
+int64_t ensure_march(vt_cloud *c, int64_t n) {
   // Cells a ray may cross: several times the mean of a uniform mesh along a
   // box diagonal; longer rays run in the engine.
   int cap = (int)(2.6 * std::cbrt((double)c->n)) + 64;
@@ -761,7 +764,6 @@ int64_t ensure_march(vt_cloud *c, int64_t n, hipStream_t st) {
     c->march.seq = dev_alloc<uint4>((size_t)cap * rays);
     c->march.c0 = dev_alloc<uint32_t>((size_t)rays);
     c->march.ctr = dev_alloc<uint32_t>(kMarchCounters);
-    HIP_OK(hipMemsetAsync(c->march.ctr, 0, kMarchCounters * sizeof(uint32_t), st));
     c->march_rays = (size_t)rays;
   }
   if (c->fall_cap < (size_t)n) {
@@ -783,7 +785,7 @@ int march(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io
   MarchCall m{};
   m.cus = num_cus(c->device);
   ensure_scratch(c, (size_t)march_locate_grid(m.cus) * kBlock);
-  const int64_t rays = ensure_march(c, n, st);
+  const int64_t rays = ensure_march(c, n);
   m.C = c->dc;
   m.S = c->scratch;
   m.N = NbLists{c->d_nb, c->d_nr2, c->d_boxes};
@@ -1258,7 +1260,7 @@ int project_noalloc(vt_cloud *c, const double *d_s, const double *d_e, int64_t n
         (int)std::min<int64_t>(64, std::max<int64_t>(1, (64 * nr + lanes - 1) / lanes));
     s.tile_row = c->ray_row;
     s.ray_order = (own_order && c->order_n == nr && nr > 0) ? c->d_order : nullptr;
-    k_clear_call<<<1, 64, 0, st>>>(c->d_err, c->d_stats);
+    k_clear_call<<<1, 64, 0, st>>>(c->d_err, c->d_stats, nullptr);
     HIP_OK(hipGetLastError());
     return grid;
   };
