@@ -13,11 +13,15 @@
  * RuntimeError).  vt_last_error() returns the message of the last failure on
  * the calling thread, with the reference's wording.
  *
- * A cloud owns per-cloud device memory: its tree, 260 bytes of neighbour lists
- * per point, and work memory kept between calls (the kernels' per-lane stacks,
- * the march's envelopes, at most 4.5 GiB, the deferred-ray list, the adjoint's
- * and field update's buffers): calls on one cloud must not overlap in time; different
- * clouds may be used from different threads at once.
+ * A cloud owns per-cloud device memory: its tree, 280 bytes of neighbour lists
+ * and boxes per point, and work memory kept between calls (the kernels' per-lane
+ * stacks, the deferred-ray list, the adjoint's and field update's buffers):
+ * calls on one cloud must not overlap in time; different clouds may be used from
+ * different threads at once.  A projection also leases up to 4.5 GiB of rows
+ * from the library, which keeps one such block per GPU until the GPU's last
+ * cloud goes.  Lists and rows are taken only where there is room and given back
+ * when an allocation of the library fails; rays run without them in the ray
+ * engine, with the same results (vt_cloud_set_march_limit bounds them).
  *
  * Cell ids crossing the boundary are indices into the filtered particle list,
  * as in the reference (PointCloud::orig_ids maps them to input rows).
@@ -267,6 +271,12 @@ typedef struct {
 } vt_view;
 int vt_grid_rays(const vt_view *views, size_t nviews, double *d_start, double *d_end,
                  void *stream);
+
+/* Device memory that the march of this cloud's rays may take (neighbour lists,
+ * boxes and rows), in bytes; lists that are larger are dropped at once.  0: every
+ * ray runs in the ray engine.  The default is SIZE_MAX.  Speed and memory only,
+ * never results.  No reference counterpart. */
+int vt_cloud_set_march_limit(vt_cloud *cloud, size_t max_bytes);
 
 /* Launch parameters of the ray kernels (process-wide): lanes of a wave that
  * run their walk steps together, lanes that run their leaf steps together

@@ -73,6 +73,7 @@ SIGNATURES = {
     "vt_project_segments": (I, [P, P, P, S, I, P, P, P, P, P, P]),
     "vt_cloud_set_fields": (I, [P, P, P]),
     "vt_cloud_set_ray_rows": (I, [P, C.c_int64]),
+    "vt_cloud_set_march_limit": (I, [P, S]),
     "vt_cloud_set_ray_order": (I, [P, P, C.c_int64, P]),
     "vt_cloud_order_rays": (I, [P, P, P, P, C.c_int64, C.c_int64, C.c_int64, P, P, P]),
     "vt_cloud_save_tree": (I, [P, P, S, C.POINTER(S)]),

@@ -259,6 +259,15 @@ class PointCloud:
     def get_ray_rows(self) -> int:
         return getattr(self, "_ray_rows", 0)
 
+    def set_march_limit(self, max_bytes: int | None) -> None:
+        """Device memory that the march of this cloud's rays may take, in bytes
+        (vt_cloud_set_march_limit); 0: every ray runs in the ray engine, None:
+        as much as there is room for.  Speed and memory only."""
+        n = C.c_size_t(-1).value if max_bytes is None else int(max_bytes)
+        if n < 0:
+            raise ValueError("max_bytes must not be negative")
+        _lib.check(_lib.lib().vt_cloud_set_march_limit(self._handle(), n))
+
     def set_ray_order(self, order: torch.Tensor | None) -> None:
         """Order in which the kernels take the rays of coming calls with
         len(order) rays: a permutation of [0, n) as an int32 device tensor,

@@ -89,7 +89,8 @@ void march_batch(const MarchCall &m, bool periodic);
 // Checks the batch's envelopes and hands their segments to `io`'s sinks.
 template <class IO>
 void march_finish(const MarchCall &m, bool periodic, const IO &io);
-// The most workgroups k_locate_far runs (its scratch is sized by it).
+// The most workgroups k_locate_far runs, as many as its stacks in LDS let the chip
+// hold (its scratch is sized by it).
 int march_locate_grid(int cus);
 
 // Records a ray's segments in one run of the pool (RecordIO for the march).

@@ -1372,7 +1372,7 @@ void march_build_boxes(const DevCloud &C, uint32_t nodes, BNode *boxes, uint32_t
   k_box_climb<<<(C.n + 255) / 256, 256, 0, st>>>(C.gen, C.n, boxes, parent, leaf_parent, arrived);
 }
 
-int march_locate_grid(int cus) { return 4 * cus; }
+int march_locate_grid(int cus) { return 2 * cus; }
 
 template <bool PER>
 static void march_batch_p(const MarchCall &m) {

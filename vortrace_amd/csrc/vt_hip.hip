@@ -25,6 +25,7 @@
 #include <cstring>
 #include <map>
 #include <mutex>
+#include <set>
 #include <stdexcept>
 #include <string>
 #include <thread>
@@ -305,11 +306,20 @@ struct HipError : std::runtime_error {
       throw HipError(std::string("HIP error in " #expr ": ") + hipGetErrorString(e_)); \
   } while (0)
 
+// Frees what marches of the current device can do without (march_memory.h);
+// false when there was nothing.
+bool reclaim_march_memory();
+
 template <class T>
 T *dev_alloc(size_t count) {
   void *p = nullptr;
   if (count == 0) count = 1;
-  HIP_OK(hipMalloc(&p, count * sizeof(T)));
+  hipError_t e = hipMalloc(&p, count * sizeof(T));
+  if (e == hipErrorOutOfMemory && reclaim_march_memory()) {
+    (void)hipGetLastError();
+    e = hipMalloc(&p, count * sizeof(T));
+  }
+  HIP_OK(e);
   return static_cast<T *>(p);
 }
 
@@ -323,6 +333,8 @@ std::string fmt(const char *f, ...) {
 }
 
 }  // namespace
+
+#include "march_memory.h"
 
 struct vt_cloud {
   // host copy (filtered order), PointCloud members of include/pointcloud.hpp:21-32
@@ -359,30 +371,25 @@ struct vt_cloud {
   int64_t order_n = 0;
   uint32_t *d_defer = nullptr;  // rays left to the K_EXPAND-capable kernels
   size_t defer_cap = 0;
-  uint32_t *d_nb = nullptr;     // neighbour lists (null: every ray runs in the engine)
-  float *d_nr2 = nullptr;
-  BNode *d_boxes = nullptr;     // and the tree's boxes
-  MarchBufs march{};            // the march's work buffers, for march_rays slots
-  size_t march_rays = 0;
-  uint32_t *d_fall = nullptr;   // rays the march left to the engine
-  size_t fall_cap = 0;
+  MarchLists lists;             // of the march (none: every ray runs in the engine)
+  size_t march_limit = SIZE_MAX;  // device memory a march may take
+  bool counted = false;         // among the device's uploaded clouds
   uint32_t *d_order_hist = nullptr;  // ray-order estimate: generators per histogram cell
   float *d_order_grid = nullptr;     // and their cube roots (built on first use)
   int kspill = 0;
+  int64_t inner_nodes = 0;
   DevCloud dc{};
   // Work buffers of the adjoint, recording and field-update calls, kept
   // between calls (slot i of a call's i-th request, grown when too small).
   std::vector<std::pair<void *, size_t>> arena;
 
   void free_device() {
+    leave_march_memory(this);
     for (void *p : {(void *)d_nodes, (void *)d_recs, (void *)d_gen, (void *)d_fields, (void *)d_slot_id,
                     (void *)d_call, (void *)scratch.knn_spill,
                     (void *)scratch.walk_tag, (void *)scratch.walk_s,
                     (void *)scratch.big_id, (void *)scratch.big_d, (void *)help_ev,
-                    (void *)help_steal, (void *)d_defer, (void *)d_nb, (void *)d_nr2,
-                    (void *)march.seq, (void *)march.c0, (void *)d_boxes,
-                    (void *)march.ctr, (void *)d_fall,
-                    (void *)d_order, (void *)d_order_hist, (void *)d_order_grid})
+                    (void *)help_steal, (void *)d_defer, (void *)d_order, (void *)d_order_hist, (void *)d_order_grid})
       if (p) (void)hipFree(p);
     d_order_hist = nullptr;
     d_order_grid = nullptr;
@@ -394,13 +401,6 @@ struct vt_cloud {
     arena.clear();
     d_defer = nullptr;
     defer_cap = 0;
-    d_nb = nullptr;
-    d_nr2 = nullptr;
-    d_boxes = nullptr;
-    march = MarchBufs{};
-    march_rays = 0;
-    d_fall = nullptr;
-    fall_cap = 0;
     d_nodes = nullptr;
     d_recs = nullptr;
     d_gen = nullptr;
@@ -418,6 +418,40 @@ struct vt_cloud {
 };
 
 namespace {
+
+bool reclaim_march_memory() {
+  int dev = -1;
+  if (hipGetDevice(&dev) != hipSuccess) return false;
+  MarchMemory &m = march_memory();
+  std::lock_guard<std::mutex> lk(m.mu);
+  bool freed = m.drop_rows(dev);
+  for (auto it = m.listed.begin(); it != m.listed.end();) {
+    vt_cloud *c = *it;
+    if (c->device == dev && c->lists.drop()) {
+      freed = true;
+      it = m.listed.erase(it);
+    } else {
+      ++it;
+    }
+  }
+  return freed;
+}
+
+void leave_march_memory(vt_cloud *c) {
+  MarchMemory &m = march_memory();
+  std::lock_guard<std::mutex> lk(m.mu);
+  m.listed.erase(c);
+  (void)c->lists.drop();
+  if (c->counted && --m.clouds[c->device] == 0) (void)m.drop_rows(c->device);
+  c->counted = false;
+}
+
+void join_march_memory(vt_cloud *c) {
+  MarchMemory &m = march_memory();
+  std::lock_guard<std::mutex> lk(m.mu);
+  if (!c->counted) ++m.clouds[c->device];
+  c->counted = true;
+}
 
 int num_cus(int dev) {
   static std::mutex mu;
@@ -551,9 +585,8 @@ __global__ void k_clear_call(ErrRec *err, Stats *stats, uint32_t *starts) {
 // One launch and one copy back a call: with two fills and two copies they were
 // a third of a 16^2 call.  Nothing a call counts in is left to an earlier one,
 // which may have failed between its launches or never run (stream capture).
-void reset_call(vt_cloud *c, hipStream_t st) {
-  k_clear_call<<<1, 64, 0, st>>>(c->d_err, c->d_stats,
-                                 c->march.ctr ? c->march.ctr + kParts : nullptr);
+void reset_call(vt_cloud *c, hipStream_t st, uint32_t *starts = nullptr) {
+  k_clear_call<<<1, 64, 0, st>>>(c->d_err, c->d_stats, starts);
   HIP_OK(hipGetLastError());
 }
 
@@ -741,56 +774,85 @@ void launch(vt_cloud *c, K kernel, int64_t n, hipStream_t st, Timer &tm, A... ar
 // lists.  Measured at 2M clustered cells, 512^2 rays: 41.0 ms in the engine,
 // 9.8 ms marched; one ray across 20k cells 1.2 against 0.2 ms.
 // help_events = 0 asks for the engine alone.
-bool march_pays(const vt_cloud *c) { return c->d_nb != nullptr && help_events() > 0; }
+bool march_pays(const vt_cloud *c) { return c->march_limit > 0 && help_events() > 0; }
 
-// The march's work buffers for at most `n` rays, in batches of what fits in
-// kMarchBytes.  Returns the batch size.
+// Builds the cloud's neighbour lists and boxes, if there is room for them.  They
+// stay until the cloud is uploaded again, or an allocation needs their memory.
+void build_lists(vt_cloud *c, hipStream_t st) {
+  if (c->n > kNbMaxPoints || !c->bounded) return;
+  const size_t nodes = (size_t)c->inner_nodes;
+  // (Each list is two whole lines.)
+  const size_t box_bytes = (nodes * sizeof(BNode) + 255) / 256 * 256;
+  const size_t nb_bytes = c->n * kNbMax * sizeof(uint32_t);
+  const size_t bytes = box_bytes + nb_bytes + c->n * sizeof(float);
+  MarchLists &l = c->lists;
+  if (bytes > c->march_limit || !l.alloc(bytes)) return;
+  l.N.boxes = static_cast<BNode *>(l.p);
+  l.N.nb = reinterpret_cast<uint32_t *>(static_cast<char *>(l.p) + box_bytes);
+  l.N.r2 = reinterpret_cast<float *>(static_cast<char *>(l.p) + box_bytes + nb_bytes);
+  uint32_t *nb = const_cast<uint32_t *>(l.N.nb);
+  // The lists' memory serves as the boxes' work space first: it holds
+  // 64 words per point, and there are fewer inner nodes than points.
+  march_build_boxes(c->dc, (uint32_t)nodes, const_cast<BNode *>(l.N.boxes), nb, st);
+  HIP_OK(hipGetLastError());
+  march_build_lists(c->dc, nb, const_cast<float *>(l.N.r2), st);
+  HIP_OK(hipGetLastError());
+  // (A build that is only recorded, under stream capture, ends here.)
+  HIP_OK(hipStreamSynchronize(st));
+  MarchMemory &m = march_memory();
+  std::lock_guard<std::mutex> lk(m.mu);
+  m.listed.insert(c);
+  l.state.store(MarchLists::kIdle);
+}
+
+// A march's work buffers for n rays, in batches of as many rays as the block of
+// rows holds: at most kMarchBytes, less when memory is short, and no march at
+// all below kMarchLeast rays a batch.
 constexpr size_t kMarchBytes = (size_t)9 << 29;  // 4.5 GiB
-int64_t ensure_march(vt_cloud *c, int64_t n) {
+constexpr int64_t kMarchLeast = 16384;
+bool take_march(vt_cloud *c, int64_t n, RowLease &rows, MarchBufs &B, uint32_t *&fall,
+                int64_t &batch) {
   // Cells a ray may cross: several times the mean of a uniform mesh along a
   // box diagonal; longer rays run in the engine.
   int cap = (int)(2.6 * std::cbrt((double)c->n)) + 64;
   cap = std::min(4096, std::max(128, (cap + 63) / 64 * 64));
-  const size_t per = (size_t)cap * sizeof(uint4);
-  const int64_t most = (int64_t)(kMarchBytes / per) / 64 * 64;
-  const int64_t batches = (n + most - 1) / most;
-  const int64_t rays = ((n + batches - 1) / batches + 63) / 64 * 64;
-  if (c->march_rays < (size_t)rays || c->march.cap != cap) {
-    for (void *p : {(void *)c->march.seq, (void *)c->march.c0, (void *)c->march.ctr})
-      if (p) (void)hipFree(p);
-    c->march = MarchBufs{};
-    c->march_rays = 0;
-    c->march.cap = cap;
-    c->march.seq = dev_alloc<uint4>((size_t)cap * rays);
-    c->march.c0 = dev_alloc<uint32_t>((size_t)rays);
-    c->march.ctr = dev_alloc<uint32_t>(kMarchCounters);
-    c->march_rays = (size_t)rays;
-  }
-  if (c->fall_cap < (size_t)n) {
-    if (c->d_fall) (void)hipFree(c->d_fall);
-    c->d_fall = nullptr;
-    c->fall_cap = 0;
-    c->d_fall = dev_alloc<uint32_t>((size_t)n);
-    c->fall_cap = (size_t)n;
-  }
-  return rays;
+  const size_t per = (size_t)cap * sizeof(uint4) + sizeof(uint32_t);
+  // The counters and the list of the rays that are left stay for all batches.
+  const size_t fixed = (size_t)n * sizeof(uint32_t) + 256;
+  const size_t held = c->lists.bytes;
+  if (held > c->march_limit) return false;
+  auto bytes = [&](int64_t rays) { return fixed + (size_t)((rays + 63) / 64 * 64) * per; };
+  const int64_t most = std::max<int64_t>(kMarchLeast, (int64_t)(kMarchBytes / per));
+  const size_t least = bytes(std::min(n, kMarchLeast));
+  const size_t want = std::min(bytes(std::min(n, most)), c->march_limit - held);
+  if (want < least || !rows.take(c->device, want, least)) return false;
+  const size_t use = std::min(rows.bytes(), want);
+  const int64_t fit = (int64_t)((use - fixed) / per) / 64 * 64;
+  const int64_t batches = (n + fit - 1) / fit;
+  batch = ((n + batches - 1) / batches + 63) / 64 * 64;
+  char *p = static_cast<char *>(rows.data());
+  B.seq = reinterpret_cast<uint4 *>(p);
+  p += (size_t)batch * cap * sizeof(uint4);
+  B.c0 = reinterpret_cast<uint32_t *>(p);
+  p += (size_t)batch * sizeof(uint32_t);
+  B.ctr = reinterpret_cast<uint32_t *>(p);
+  fall = B.ctr + 64;
+  B.cap = cap;
+  return true;
 }
 
 // Marches n rays and hands their segments to io; *fallback rays are left, in
-// c->d_fall, to the engine.
+// `fall`, to the engine.
 template <class IO>
 int march(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io, hipStream_t st,
-          int64_t *fallback) {
-  if (n > 0xFFFFFFFFll) return fail(VT_EINVAL, "at most 2^32 - 1 rays per call");
+          const MarchBufs &B, uint32_t *fall, int64_t batch, int64_t *fallback) {
   MarchCall m{};
   m.cus = num_cus(c->device);
-  ensure_scratch(c, (size_t)march_locate_grid(m.cus) * kBlock);
-  const int64_t rays = ensure_march(c, n);
   m.C = c->dc;
   m.S = c->scratch;
-  m.N = NbLists{c->d_nb, c->d_nr2, c->d_boxes};
-  m.B = c->march;
-  m.fall = c->d_fall;
+  m.N = c->lists.N;
+  m.B = B;
+  m.fall = fall;
   m.err = c->d_err;
   m.stats = c->d_stats;
   m.pool = 8 * help_events();
@@ -802,12 +864,12 @@ int march(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io
   m.R.tile_n = m.R.tile_row ? (uint32_t)((uint64_t)n / (8ull * m.R.tile_row) *
                                          (8ull * m.R.tile_row))
                             : 0u;
-  reset_call(c, st);
+  reset_call(c, st, B.ctr + kParts);
   Timer tm;
   HIP_OK(hipEventRecord(tm.e0, st));
-  for (int64_t base = 0; base < n; base += rays) {
+  for (int64_t base = 0; base < n; base += batch) {
     m.R.base = base;
-    m.R.n = std::min(rays, n - base);
+    m.R.n = std::min(batch, n - base);
     march_batch(m, c->periodic);
     HIP_OK(hipGetLastError());
     march_finish(m, c->periodic, io);
@@ -858,15 +920,28 @@ bool engine_sooner(vt_cloud *c, const double *s, const double *e, int64_t n, hip
 template <class IO, class Fast, class Slow>
 int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io,
                hipStream_t st, Fast &&fast, Slow &&slow, bool projects = false) {
+  if (n > 0xFFFFFFFFll) return fail(VT_EINVAL, "at most 2^32 - 1 rays per call");
   const uint32_t *list = nullptr;
   int64_t left = n;
+  bool marched = false;
+  RowLease rows(st);
   // (The kernels that count and list segments are slower than the march for any
   // number of rays.)
-  const bool marched = march_pays(c) && !(projects && engine_sooner(c, s, e, n, st));
-  if (marched) {
-    const int rc = march(c, s, e, n, io, st, &left);
-    if (rc || left == 0) return rc;
-    list = c->d_fall;
+  if (march_pays(c)) {
+    // (The march's own searches run on the engine's lanes.)
+    ensure_scratch(c, (size_t)march_locate_grid(num_cus(c->device)) * kBlock);
+    MarchBufs B{};
+    uint32_t *fall = nullptr;
+    int64_t batch = 0;
+    const ListLease lists(c->lists);
+    if (lists && !(projects && engine_sooner(c, s, e, n, st)) &&
+        take_march(c, n, rows, B, fall, batch)) {
+      const int rc = march(c, s, e, n, io, st, B, fall, batch, &left);
+      rows.idle();  // (the call has been waited for)
+      if (rc || left == 0) return rc;
+      marched = true;
+      list = fall;
+    }
   }
   return two_pass(
       c, st, (size_t)left, [&](Timer &tm) { fast(tm, list, left); },
@@ -1490,31 +1565,9 @@ int vt_cloud_upload(vt_cloud *c) {
     d.periodic = c->periodic;
     d.root = dt.root;
     d.rroot = dt.rroot;
-    // Neighbour lists for the march; without room for them every ray runs in
-    // the engine.  So it does through a tree that does not bound its points:
-    // searches then find what the cuts let them, which only the engine repeats.
-    if (c->n <= kNbMaxPoints && c->bounded) {
-      const size_t nn = dt.nodes.size();
-      void *nb = nullptr, *nr = nullptr, *bx = nullptr;
-      if (hipMalloc(&nb, c->n * kNbMax * sizeof(uint32_t)) == hipSuccess &&
-          hipMalloc(&nr, c->n * sizeof(float)) == hipSuccess &&
-          hipMalloc(&bx, std::max<size_t>(1, nn) * sizeof(BNode)) == hipSuccess) {
-        c->d_nb = static_cast<uint32_t *>(nb);
-        c->d_nr2 = static_cast<float *>(nr);
-        c->d_boxes = static_cast<BNode *>(bx);
-        // The lists' memory serves as the boxes' work space first: it holds
-        // 64 words per point, and there are fewer inner nodes than points.
-        march_build_boxes(d, (uint32_t)nn, c->d_boxes, c->d_nb, nullptr);
-        HIP_OK(hipGetLastError());
-        march_build_lists(d, c->d_nb, c->d_nr2, nullptr);
-        HIP_OK(hipGetLastError());
-        HIP_OK(hipStreamSynchronize(nullptr));
-      } else {
-        (void)hipGetLastError();
-        for (void *p : {nb, nr, bx})
-          if (p) (void)hipFree(p);
-      }
-    }
+    c->inner_nodes = (int64_t)dt.nodes.size();
+    join_march_memory(c);
+    build_lists(c, nullptr);
     c->tree_built = true;
     return VT_OK;
   });
@@ -1892,6 +1945,19 @@ int vt_cloud_set_ray_rows(vt_cloud *c, int64_t row) {
   if (row < 0 || row > 0x7FFFFFFF) return fail(VT_EINVAL, "row length out of range [0, 2^31)");
   c->ray_row = (uint32_t)row;
   return VT_OK;
+}
+
+int vt_cloud_set_march_limit(vt_cloud *c, size_t max_bytes) {
+  return guarded([&]() -> int {
+    if (!c) return fail(VT_EINVAL, "null cloud");
+    c->march_limit = max_bytes;
+    if (c->lists.bytes > max_bytes) {
+      MarchMemory &m = march_memory();
+      std::lock_guard<std::mutex> lk(m.mu);
+      if (c->lists.drop()) m.listed.erase(c);
+    }
+    return VT_OK;
+  });
 }
 
 int vt_cloud_set_ray_order(vt_cloud *c, const uint32_t *d_order, int64_t n, void *stream) {
