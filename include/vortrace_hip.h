@@ -19,7 +19,8 @@
  * calls on one cloud must not overlap in time; different clouds may be used from
  * different threads at once.  A projection also leases up to 4.5 GiB of rows
  * from the library, which keeps one such block per GPU until the GPU's last
- * cloud goes.  Lists and rows are taken only where there is room and given back
+ * cloud goes.  Lists are built by the first projections that are worth it.  Lists
+ * and rows are taken only where there is room and given back
  * when an allocation of the library fails; rays run without them in the ray
  * engine, with the same results (vt_cloud_set_march_limit bounds them).
  *

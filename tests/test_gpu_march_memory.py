@@ -132,3 +132,26 @@ def test_threads_share_rows():
     for t in threads:
         t.join()
     assert not bad
+
+
+def test_lists_wait_for_rays_that_pay_for_them():
+    """A cloud that is uploaded and queried holds its tree alone; a few rays run
+    without lists until they have cost as much, with the same bits throughout."""
+    n = 1_000_000
+    pos, rho = synthetic.uniform_mesh(n, seed=99)
+    cloud = vt.PointCloud()
+    cloud.loadPoints(pos, rho, BB, periodic=True)
+    torch.cuda.synchronize()
+    free0 = torch.cuda.mem_get_info()[0]
+    cloud.buildTree()
+    _say("queries")
+    ids, _ = cloud.query_tensor(torch.rand(1000, 3, dtype=torch.float64) * 100.0, 2)
+    assert ids.shape == (1000, 2)
+    assert free0 - torch.cuda.mem_get_info()[0] < 200 * n + (1 << 30), "lists before any ray"
+    s, e = _grid(3, 5)
+    p = vt.Projection(s, e)
+    first = p.project_tensor(cloud)
+    free1 = torch.cuda.mem_get_info()[0]
+    for _ in range(40):
+        assert torch.equal(p.project_tensor(cloud), first)
+    assert free1 - torch.cuda.mem_get_info()[0] > 200 * n, "no lists after forty calls"

@@ -2,7 +2,8 @@
 // ray runs in the ray engine.  So it is taken only where there is room, and given
 // back when an allocation that a call cannot do without fails.
 //
-//  * Lists and boxes (280 B per cell) belong to their cloud.
+//  * Lists and boxes (280 B per cell) belong to their cloud and are built by the
+//    first calls that are worth it.
 //  * Rows (up to 4.5 GiB while a call marches) belong to no cloud: a call leases a
 //    block and returns it when it has been waited for.  One block per device is
 //    kept between calls, until its last cloud goes.
@@ -29,8 +30,10 @@ struct MarchLists {
   void *p = nullptr;  // one allocation, which N points into
   size_t bytes = 0;
   vt::NbLists N{};
+  bool ready() const { return state.load() != kNone; }
   // Lists stay for their cloud's life, so they may take half of what is free.
   bool alloc(size_t want) {
+    if (p && bytes >= want) return true;  // (from a build that failed half way)
     if (want > free_for(want) / 2 || hipMalloc(&p, want) != hipSuccess) {
       (void)hipGetLastError();
       p = nullptr;
@@ -81,7 +84,7 @@ void leave_march_memory(vt_cloud *c);
 struct ListLease {
   MarchLists &l;
   const bool held;
-  explicit ListLease(MarchLists &lists) : l(lists), held(take(lists)) {}
+  ListLease(MarchLists &lists, bool wanted) : l(lists), held(wanted && take(lists)) {}
   ListLease(const ListLease &) = delete;
   ~ListLease() {
     if (held) l.state.store(MarchLists::kIdle);

@@ -372,6 +372,7 @@ struct vt_cloud {
   uint32_t *d_defer = nullptr;  // rays left to the K_EXPAND-capable kernels
   size_t defer_cap = 0;
   MarchLists lists;             // of the march (none: every ray runs in the engine)
+  double engine_ms = 0.0;       // spent without lists so far (lists_pay)
   size_t march_limit = SIZE_MAX;  // device memory a march may take
   bool counted = false;         // among the device's uploaded clouds
   uint32_t *d_order_hist = nullptr;  // ray-order estimate: generators per histogram cell
@@ -776,9 +777,24 @@ void launch(vt_cloud *c, K kernel, int64_t n, hipStream_t st, Timer &tm, A... ar
 // help_events = 0 asks for the engine alone.
 bool march_pays(const vt_cloud *c) { return c->march_limit > 0 && help_events() > 0; }
 
+// Whether the cloud's lists are worth building for a call of n rays: once the
+// calls that ran without them, this one included, have cost the engine what the
+// lists cost to build.  So a cloud that is only queried or sliced, or projects a
+// few rays once, has none.  Lists take .35 ms at 5k cells, 2.4 to 4.3 at 200k and
+// 12 at 2M clustered ones; calls without them .6 ms (one ray, 20k cells), 2.8
+// (128^2, 100k), 41 (512^2, 2M).  Building a cloud and its first projection,
+// lists at upload -> here: 5k cells, 16^2 rays 1.68 -> 1.71 ms, 100k, 128^2
+// 15.96 -> 15.68; building alone 1.05 -> .71 and 14.5 -> 13.7.
+bool lists_pay(const vt_cloud *c, int64_t n) {
+  const double build_ms = 0.3 + 1e-5 * (double)c->n;
+  const double call_ms = 0.6 + 1.5e-6 * (double)n * 1.1 * std::cbrt((double)c->n);
+  return c->engine_ms + call_ms >= build_ms;
+}
+
 // Builds the cloud's neighbour lists and boxes, if there is room for them.  They
 // stay until the cloud is uploaded again, or an allocation needs their memory.
 void build_lists(vt_cloud *c, hipStream_t st) {
+  c->engine_ms = 0.0;  // (without room, or once dropped, they are due again later)
   if (c->n > kNbMaxPoints || !c->bounded) return;
   const size_t nodes = (size_t)c->inner_nodes;
   // (Each list is two whole lines.)
@@ -927,25 +943,30 @@ int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const I
   RowLease rows(st);
   // (The kernels that count and list segments are slower than the march for any
   // number of rays.)
-  if (march_pays(c)) {
-    // (The march's own searches run on the engine's lanes.)
-    ensure_scratch(c, (size_t)march_locate_grid(num_cus(c->device)) * kBlock);
-    MarchBufs B{};
-    uint32_t *fall = nullptr;
-    int64_t batch = 0;
-    const ListLease lists(c->lists);
-    if (lists && !(projects && engine_sooner(c, s, e, n, st)) &&
-        take_march(c, n, rows, B, fall, batch)) {
-      const int rc = march(c, s, e, n, io, st, B, fall, batch, &left);
-      rows.idle();  // (the call has been waited for)
-      if (rc || left == 0) return rc;
-      marched = true;
-      list = fall;
+  const bool wants = march_pays(c);
+  if (wants && !c->lists.ready() && lists_pay(c, n)) build_lists(c, st);
+  {
+    const ListLease lists(c->lists, wants);
+    if (lists && !(projects && engine_sooner(c, s, e, n, st))) {
+      // (The march's own searches run on the engine's lanes.)
+      ensure_scratch(c, (size_t)march_locate_grid(num_cus(c->device)) * kBlock);
+      MarchBufs B{};
+      uint32_t *fall = nullptr;
+      int64_t batch = 0;
+      if (take_march(c, n, rows, B, fall, batch)) {
+        const int rc = march(c, s, e, n, io, st, B, fall, batch, &left);
+        rows.idle();  // (the call has been waited for)
+        if (rc || left == 0) return rc;
+        marched = true;
+        list = fall;
+      }
     }
   }
-  return two_pass(
+  const int rc = two_pass(
       c, st, (size_t)left, [&](Timer &tm) { fast(tm, list, left); },
       [&](Timer &tm, int64_t nd) { slow(tm, nd); }, marched);
+  if (wants && !c->lists.ready()) c->engine_ms += g_stats.kernel_ms;
+  return rc;
 }
 
 template <int MODE, int NF>
@@ -1566,8 +1587,8 @@ int vt_cloud_upload(vt_cloud *c) {
     d.root = dt.root;
     d.rroot = dt.rroot;
     c->inner_nodes = (int64_t)dt.nodes.size();
+    c->engine_ms = 0.0;
     join_march_memory(c);
-    build_lists(c, nullptr);
     c->tree_built = true;
     return VT_OK;
   });
