@@ -320,6 +320,15 @@ typedef struct {
 } vt_call_stats;
 int vt_last_call_stats(vt_call_stats *out);
 
+/* How that call was marched: rays marched (0: every ray ran in the ray engine),
+ * those of them left to the engine, and the intervals of the march's check that
+ * lanes took from one another and handed back (counted in vt_call_stats too;
+ * the rest there is the engine's). */
+typedef struct {
+  int64_t rays, left, intervals, intervals_back;
+} vt_march_stats;
+int vt_last_march_stats(vt_march_stats *out);
+
 #ifdef __cplusplus
 }
 #endif

@@ -41,6 +41,11 @@ class CallStats(C.Structure):
                 ("intervals_back", C.c_int64)]
 
 
+class MarchStats(C.Structure):
+    _fields_ = [("rays", C.c_int64), ("left", C.c_int64), ("intervals", C.c_int64),
+                ("intervals_back", C.c_int64)]
+
+
 WARN_FN = C.CFUNCTYPE(None, C.c_char_p, C.c_void_p)
 
 # name -> (restype, argtypes); every symbol include/vortrace_hip.h declares.
@@ -87,6 +92,7 @@ SIGNATURES = {
     "vt_set_tuning": (I, [C.POINTER(Tuning)]),
     "vt_get_tuning": (I, [C.POINTER(Tuning)]),
     "vt_last_call_stats": (I, [C.POINTER(CallStats)]),
+    "vt_last_march_stats": (I, [C.POINTER(MarchStats)]),
     "vt_cloud_lanes": (I, [P, I, I, C.POINTER(C.c_int64)]),
 }
 
@@ -134,4 +140,10 @@ def check(rc: int) -> None:
 def last_call_stats() -> CallStats:
     st = CallStats()
     check(lib().vt_last_call_stats(C.byref(st)))
+    return st
+
+
+def last_march_stats() -> MarchStats:
+    st = MarchStats()
+    check(lib().vt_last_march_stats(C.byref(st)))
     return st

@@ -277,6 +277,7 @@ namespace {
 
 thread_local std::string g_err;
 thread_local vt_call_stats g_stats{};
+thread_local vt_march_stats g_march{};
 std::mutex g_warn_mu;
 vt_warning_fn g_warn_fn = nullptr;
 void *g_warn_user = nullptr;
@@ -604,7 +605,10 @@ int finish_call(vt_cloud *c, hipStream_t st, hipEvent_t e0, hipEvent_t e1, bool 
   const Stats &ss = call.stats;
   float ms = 0;
   if (e0 && e1) HIP_OK(hipEventElapsedTime(&ms, e0, e1));
-  if (!more) g_stats = vt_call_stats{};
+  if (!more) {
+    g_stats = vt_call_stats{};
+    g_march = vt_march_stats{};
+  }
   if (fallback) *fallback = (int64_t)ss.fallback;
   g_stats.segments += (int64_t)ss.segments;
   g_stats.queries += (int64_t)ss.queries;
@@ -894,6 +898,7 @@ int march(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io
   HIP_OK(hipEventRecord(tm.e1, st));
   const int rc = finish_call(c, st, tm.e0, tm.e1, false, fallback);
   g_stats.queries += n;  // the start cells' searches
+  g_march = vt_march_stats{n, *fallback, g_stats.intervals, g_stats.intervals_back};
   return rc;
 }
 
@@ -2209,6 +2214,7 @@ int vt_adjoint_recorded(const vt_cloud *cc, size_t nrays, int mode, const int64_
     hipStream_t st = static_cast<hipStream_t>(stream);
     HIP_OK(hipMemsetAsync(d_grad_fields, 0, c->n * c->nf * sizeof(double), st));
     g_stats = vt_call_stats{};
+    g_march = vt_march_stats{};
     if (nrays == 0) return VT_OK;
     const int64_t n = (int64_t)nrays;
     DevBufs B(c);
@@ -2330,6 +2336,12 @@ int vt_cloud_lanes(const vt_cloud *cc, int mode, int recorded, int64_t *lanes) {
     }
     return VT_OK;
   });
+}
+
+int vt_last_march_stats(vt_march_stats *out) {
+  if (!out) return fail(VT_EINVAL, "null argument");
+  *out = g_march;
+  return VT_OK;
 }
 
 int vt_last_call_stats(vt_call_stats *out) {
