@@ -110,3 +110,32 @@ def test_recorded_forward(tuning):
         res.append((img.detach(), f.grad))
     for img, grad in res[1:]:
         assert torch.equal(img, res[0][0]) and torch.equal(grad, res[0][1])
+
+
+def test_left_rays_are_walked_once(tuning):
+    """Rays of some 240 cells, 160 of them in a dense slab, many left by the march:
+    an interval that its walker has no room for is handed back and walked again,
+    by every giver above it, so the leftovers need room for whole intervals."""
+    rng = np.random.default_rng(17)
+    h = 2e-3
+    g = np.stack(np.meshgrid(np.arange(24), np.arange(24), np.arange(110), indexing="ij"), -1)
+    slab = 50.0 + h * (g.reshape(-1, 3) + 0.25 + 0.5 * rng.random((24 * 24 * 110, 3)))
+    pos = np.concatenate([slab, 100.0 * rng.random((400_000, 3))])
+    pc = vt.ProjectionCloud(pos, rng.random(len(pos)), boundbox=BB, periodic=True)
+    x = 50.0 + h * (2.0 + 20.0 * (np.arange(64) + 0.5) / 64)
+    xy = np.stack(np.meshgrid(x, x, indexing="ij"), -1).reshape(-1, 2)
+    s = torch.from_numpy(np.column_stack([xy, np.zeros(4096)])).cuda()
+    e = s + torch.tensor([0.0, 0.0, 100.0], dtype=torch.float64, device="cuda")
+    for _ in range(40):  # until the lists are built
+        got = pc.projection_tensor(s, e)
+        m = _lib.last_march_stats()
+        if m.rays:
+            break
+    st = _lib.last_call_stats()
+    given, back = st.intervals - m.intervals, st.intervals_back - m.intervals_back
+    _say(f"  {m.left} of {m.rays} rays left, {given} intervals given, {back} handed back")
+    assert m.left >= 512, "fewer rays than workgroups"
+    assert 200 <= st.segments / len(s) <= 300, "rays of other lengths than meant"
+    assert given > 0 and back == 0
+    vt.tuning.set_tuning(help_events=0)
+    assert torch.equal(pc.projection_tensor(s, e), got)

@@ -135,6 +135,29 @@ struct RowLease {
     dev = device;
     return true;
   }
+  // Makes the block at least `want` bytes up to `tail`, whose `keep` bytes are
+  // kept (tail may move); false when there is no room.  The call has been waited
+  // for.
+  bool grow(size_t want, uint32_t *&tail, size_t keep) {
+    if ((size_t)(reinterpret_cast<char *>(tail) - static_cast<char *>(b.p)) >= want) return true;
+    void *p = nullptr;
+    if (want + keep > free_for(want + keep) / 4 || hipMalloc(&p, want + keep) != hipSuccess) {
+      (void)hipGetLastError();
+      return false;
+    }
+    uint32_t *moved = reinterpret_cast<uint32_t *>(static_cast<char *>(p) + want);
+    const bool ok = hipMemcpyAsync(moved, tail, keep, hipMemcpyDeviceToDevice, st) == hipSuccess &&
+                    hipStreamSynchronize(st) == hipSuccess;
+    if (!ok) {
+      (void)hipGetLastError();
+      (void)hipFree(p);
+      return false;
+    }
+    (void)hipFree(b.p);
+    b = MarchMemory::Block{p, want + keep};
+    tail = moved;
+    return true;
+  }
   ~RowLease() {
     if (!b.p) return;
     if (busy) (void)hipStreamSynchronize(st);

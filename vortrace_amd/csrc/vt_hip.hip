@@ -366,6 +366,8 @@ struct vt_cloud {
   Scratch scratch{};
   size_t scratch_lanes = 0;
   uint4 *help_ev = nullptr, *help_steal = nullptr;  // interval buffers (scratch_lanes lanes)
+  uint4 *left_ev = nullptr;     // larger ones for the rays a march left, while they run
+  size_t left_events = 0;
   uint32_t ray_row = 0;         // rays per image row of the coming calls (0 = no image)
   uint32_t *d_order = nullptr;  // a caller's ray order for calls of order_n rays
   size_t order_cap = 0;
@@ -758,15 +760,25 @@ void launch(vt_cloud *c, K kernel, int64_t n, hipStream_t st, Timer &tm, A... ar
   c->scratch.ray_order = (c->order_n == n && n > 0) ? c->d_order : nullptr;
   Scratch s = c->scratch;
   int blocks = grid;
-  if (n > 0 && n < grid && s.help_ev) {
-    // A few rays (a march's leftovers): a workgroup each, which share the
-    // interval buffers of all lanes.  A gift of more cells than its walker has
-    // room for is walked twice, and again by every giver above: of a ray of 358
-    // cells in 128-event buffers, 5,500 queries instead of 717.
-    blocks = (int)n;
+  const bool few = n > 0 && n < grid;
+  if (s.help_ev && (few || c->left_ev)) {
+    // A gift of more cells than its walker has room for is walked twice, and
+    // again by every giver above: of a ray of 358 cells in 128-event buffers,
+    // 5,500 queries instead of 717.  So a few rays run a workgroup each and
+    // share the buffers of all lanes, and a march's leftovers use its rows where
+    // these hold more: 6,437 of 256^2 rays through a clump of a 2M mesh 65 ms in
+    // 128-event buffers, 9.5 in 448-event ones.
+    size_t events = (size_t)kHelpEvents * c->scratch_lanes;
+    if (c->left_events > events) {
+      s.help_ev = c->left_ev;
+      events = c->left_events;
+    }
+    if (few) blocks = (int)n;
     s.lanes = blocks * kBlock;
     const size_t more = c->scratch_lanes / (size_t)s.lanes;
-    s.help_cap = (int)std::min<size_t>(kHsMaxEvents, s.help_cap * more);
+    // (help_events says which part of a lane's share it may fill.)
+    s.help_cap = (int)std::min<size_t>(kHsMaxEvents,
+                                       events / (size_t)s.lanes * s.help_cap / kHelpEvents);
     s.help_steal_cap = (int)std::min<size_t>(256, s.help_steal_cap * more);
   }
   HIP_OK(hipEventRecord(tm.e0, st));
@@ -963,13 +975,33 @@ int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const I
         rows.idle();  // (the call has been waited for)
         if (rc || left == 0) return rc;
         marched = true;
+        // Buffers for the intervals of the rays that are left, once these are
+        // more than run a workgroup each: all the cells of a ray that the march
+        // has room for, 256 at least.
+        const size_t want = c->scratch_lanes * std::max(256, B.cap) * sizeof(uint4);
+        if (help_events() > 0 && left >= 2ll * num_cus(c->device) &&
+            want < c->march_limit - c->lists.bytes)
+          (void)rows.grow(want, fall, (size_t)left * sizeof(uint32_t));
+        c->left_ev = static_cast<uint4 *>(rows.data());
+        c->left_events = (size_t)(reinterpret_cast<char *>(fall) - static_cast<char *>(rows.data())) /
+                         sizeof(uint4);
         list = fall;
       }
     }
   }
+  // (The rows are given back on every way out, so the buffers in them are too.)
+  struct Gifts {
+    vt_cloud *c;
+    ~Gifts() {
+      c->left_ev = nullptr;
+      c->left_events = 0;
+    }
+  } gifts{c};
+  rows.busy = marched;
   const int rc = two_pass(
       c, st, (size_t)left, [&](Timer &tm) { fast(tm, list, left); },
       [&](Timer &tm, int64_t nd) { slow(tm, nd); }, marched);
+  rows.idle();
   if (wants && !c->lists.ready()) c->engine_ms += g_stats.kernel_ms;
   return rc;
 }
