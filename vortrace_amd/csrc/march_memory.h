@@ -135,13 +135,13 @@ struct RowLease {
     dev = device;
     return true;
   }
-  // Makes the block at least `want` bytes up to `tail`, whose `keep` bytes are
-  // kept (tail may move); false when there is no room.  The call has been waited
-  // for.
-  bool grow(size_t want, uint32_t *&tail, size_t keep) {
+  // Makes the block at least `want` bytes up to its `tail` of `size` bytes, whose
+  // first `keep` are kept (it may move); false when there is no room.  The call
+  // has been waited for.
+  bool grow(size_t want, uint32_t *&tail, size_t size, size_t keep) {
     if ((size_t)(reinterpret_cast<char *>(tail) - static_cast<char *>(b.p)) >= want) return true;
     void *p = nullptr;
-    if (want + keep > free_for(want + keep) / 4 || hipMalloc(&p, want + keep) != hipSuccess) {
+    if (want + size > free_for(want + size) / 4 || hipMalloc(&p, want + size) != hipSuccess) {
       (void)hipGetLastError();
       return false;
     }
@@ -154,7 +154,7 @@ struct RowLease {
       return false;
     }
     (void)hipFree(b.p);
-    b = MarchMemory::Block{p, want + keep};
+    b = MarchMemory::Block{p, want + size};
     tail = moved;
     return true;
   }

@@ -862,13 +862,13 @@ bool take_march(vt_cloud *c, int64_t n, RowLease &rows, MarchBufs &B, uint32_t *
   const int64_t fit = (int64_t)((use - fixed) / per) / 64 * 64;
   const int64_t batches = (n + fit - 1) / fit;
   batch = ((n + batches - 1) / batches + 63) / 64 * 64;
+  // The counters and the list at the block's end: all before them can serve the
+  // rays that are left as buffers (launch).
   char *p = static_cast<char *>(rows.data());
   B.seq = reinterpret_cast<uint4 *>(p);
-  p += (size_t)batch * cap * sizeof(uint4);
-  B.c0 = reinterpret_cast<uint32_t *>(p);
-  p += (size_t)batch * sizeof(uint32_t);
-  B.ctr = reinterpret_cast<uint32_t *>(p);
-  fall = B.ctr + 64;
+  B.c0 = reinterpret_cast<uint32_t *>(p + (size_t)batch * cap * sizeof(uint4));
+  fall = reinterpret_cast<uint32_t *>(p + rows.bytes() / 4 * 4) - n;
+  B.ctr = fall - 64;
   B.cap = cap;
   return true;
 }
@@ -981,7 +981,8 @@ int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const I
         const size_t want = c->scratch_lanes * std::max(256, B.cap) * sizeof(uint4);
         if (help_events() > 0 && left >= 2ll * num_cus(c->device) &&
             want < c->march_limit - c->lists.bytes)
-          (void)rows.grow(want, fall, (size_t)left * sizeof(uint32_t));
+          (void)rows.grow(want, fall, (size_t)n * sizeof(uint32_t),
+                          (size_t)left * sizeof(uint32_t));
         c->left_ev = static_cast<uint4 *>(rows.data());
         c->left_events = (size_t)(reinterpret_cast<char *>(fall) - static_cast<char *>(rows.data())) /
                          sizeof(uint4);
