@@ -107,3 +107,30 @@ def test_own_tree_loaded_is_marched():
         except ValueError:  # searches through such a tree may find nothing
             pass
         assert _lib.last_march_stats().rays == 0
+
+
+@pytest.mark.filterwarnings("ignore::UserWarning")
+@pytest.mark.parametrize("cells,box,rays,marched", [
+    (200, 1.0, 500, False), (300, 1.0, 500, True),          # cells large against the box
+    (200_000, 100.0, 1000, True), (200_000, 1.0, 1000, False),  # a ray or two would be left
+    (200_000, 1.0, 8192, False), (200_000, 1.0, 8193, True),    # (32 rays per CU, 256 CUs)
+    (200_000, 1.0, 100, True), (100_000, 0.03, 20_000, False)])  # next to none; most
+def test_where_a_march_does_not_pay(cells, box, rays, marched):
+    """Both sides of march_pays's lines, in periodic boxes."""
+    pos, rho = synthetic.uniform_mesh(cells, seed=63)
+    pc = vt.ProjectionCloud(box * (pos / 100.0), rho, boundbox=[0.0, box] * 3, periodic=True)
+    if cells >= 200_000:
+        assert _routes(pc, *_axis(20_000, 1, box))[0] == 20_000  # the lists are built
+    assert _routes(pc, *_axis(rays, 2, box))[0] == (rays if marched else 0)
+
+
+def test_lattice_is_left():
+    """Split points on the cells' faces: every ray is left, in the order it had."""
+    g = (np.arange(24) + 0.5) / 24
+    pos = np.stack(np.meshgrid(g, g, g, indexing="ij"), -1).reshape(-1, 3)
+    pc = vt.ProjectionCloud(pos, np.random.default_rng(1).random(len(pos)) + 0.5,
+                            boundbox=[0.0, 1.0] * 3, vol=np.full(len(pos), 24.0 ** -3))
+    x = (np.arange(100) + 0.5) / 100
+    xy = np.stack(np.meshgrid(x, x, indexing="ij"), -1).reshape(-1, 2)
+    z = np.zeros(len(xy))
+    assert _routes(pc, np.column_stack([xy, z]), np.column_stack([xy, z + 1.0])) == (10_000, 10_000)

@@ -787,11 +787,42 @@ void launch(vt_cloud *c, K kernel, int64_t n, hipStream_t st, Timer &tm, A... ar
   HIP_OK(hipEventRecord(tm.e1, st));
 }
 
-// Whether a call's rays are marched first (march.h): whenever the cloud has
-// lists.  Measured at 2M clustered cells, 512^2 rays: 41.0 ms in the engine,
-// 9.8 ms marched; one ray across 20k cells 1.2 against 0.2 ms.
-// help_events = 0 asks for the engine alone.
-bool march_pays(const vt_cloud *c) { return c->march_limit > 0 && help_events() > 0; }
+// Whether a call's n rays are marched first (march.h).  Measured at 2M clustered
+// cells, 512^2 rays: 41.0 ms in the engine, 9.8 ms marched; one ray across 20k
+// cells 1.2 against 0.2 ms.  help_events = 0 asks for the engine alone.
+//
+// A march that leaves its rays to the engine costs both.  It leaves
+//  * rays through cells that are large against a periodic box (`far` in
+//    march_batch_p): nearly all of them when cells are .21 of the box apart, a
+//    third at .15, none at .1.  4,096 rays, in the engine and marched: 100 cells
+//    .74 and .90 ms, 300 .78 and .80, 1,000 .87 and .73;
+//  * rays that meet a third generator within the clearance of a boundary.  Around
+//    every edge of a cell that is a strip of clearance / spacing, so a crossing
+//    meets one with a probability of some 13 clearance / spacing^2, and a ray
+//    through a box of N cells in 13 clearance N / area crossings, however the
+//    cells cluster.  (Measured shares, 4e-6 to .13, agree: 2M cells in boxes of
+//    100, 10 and 1, 200k and 20k in boxes of 1 and .1.)  Where that is most rays,
+//    none are marched.  With too few rays to fill the card the leftover's own
+//    walk comes on top, so there one such ray is too much: 200k cells in a unit
+//    box, 32^2 rays 1.3 ms in the engine, 2.2 marched with one ray left, 64^2 2.1
+//    and 3.2, 128^2 4.5 and 3.8.
+bool march_pays(const vt_cloud *c, int64_t n) {
+  if (c->march_limit == 0 || help_events() <= 0) return false;
+  const DevCloud &d = c->dc;
+  double side[3], scale = 0.0;
+  for (int k = 0; k < 3; ++k) {
+    side[k] = c->periodic ? d.box[k] : d.rb_hi[k] - d.rb_lo[k];
+    scale = std::max(scale, std::max(std::fabs(d.rb_lo[k]), std::fabs(d.rb_hi[k])) + d.box[k]);
+  }
+  std::sort(side, side + 3);
+  const double cells = (double)c->n;
+  if (c->periodic && std::cbrt(side[0] * side[1] * side[2] / cells) > 0.16 * side[0]) return false;
+  const double clearance = 1.05 * kTol + 1e-14 * scale * scale;
+  const double area = side[1] * side[2];
+  if (!(area > 0.0)) return true;
+  const double met = 13.0 * clearance * cells / area;
+  return met < 1.0 && (n > 32ll * num_cus(c->device) || met * (double)n < 0.5);
+}
 
 // Whether the cloud's lists are worth building for a call of n rays: once the
 // calls that ran without them, this one included, have cost the engine what the
@@ -960,7 +991,7 @@ int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const I
   RowLease rows(st);
   // (The kernels that count and list segments are slower than the march for any
   // number of rays.)
-  const bool wants = march_pays(c);
+  const bool wants = march_pays(c, n);
   if (wants && !c->lists.ready() && lists_pay(c, n)) build_lists(c, st);
   {
     const ListLease lists(c->lists, wants);
@@ -986,7 +1017,8 @@ int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const I
         c->left_ev = static_cast<uint4 *>(rows.data());
         c->left_events = (size_t)(reinterpret_cast<char *>(fall) - static_cast<char *>(rows.data())) /
                          sizeof(uint4);
-        list = fall;
+        // (All of them keep the order they would have had without a march.)
+        list = left < n ? fall : nullptr;
       }
     }
   }
