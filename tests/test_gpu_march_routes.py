@@ -114,6 +114,7 @@ def test_own_tree_loaded_is_marched():
     (200, 1.0, 500, False), (300, 1.0, 500, True),          # cells large against the box
     (200_000, 100.0, 1000, True), (200_000, 1.0, 1000, False),  # a ray or two would be left
     (200_000, 1.0, 8192, False), (200_000, 1.0, 8193, True),    # (32 rays per CU, 256 CUs)
+    (600_000, 1.0, 2900, False), (600_000, 1.0, 3100, True),    # (7e6 rays x cells per CU)
     (200_000, 1.0, 100, True), (100_000, 0.03, 20_000, False)])  # next to none; most
 def test_where_a_march_does_not_pay(cells, box, rays, marched):
     """Both sides of march_pays's lines, in periodic boxes."""
@@ -134,3 +135,13 @@ def test_lattice_is_left():
     xy = np.stack(np.meshgrid(x, x, indexing="ij"), -1).reshape(-1, 2)
     z = np.zeros(len(xy))
     assert _routes(pc, np.column_stack([xy, z]), np.column_stack([xy, z + 1.0])) == (10_000, 10_000)
+
+
+def test_rows_of_more_than_640_cells():
+    """Clouds of more than 11M cells: rows of 704 cells, 512 intervals a wave in the
+    march's check."""
+    n = 11_500_000
+    pos, rho = synthetic.uniform_mesh(n, seed=65)
+    pc = vt.ProjectionCloud(pos, rho, boundbox=BB, periodic=True)
+    marched, left = _routes(pc, *_axis(500_000, 3))
+    assert marched == 500_000 and left < 500  # (some ten meet a near-tie)

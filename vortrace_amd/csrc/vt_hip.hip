@@ -803,9 +803,12 @@ void launch(vt_cloud *c, K kernel, int64_t n, hipStream_t st, Timer &tm, A... ar
 //    cells cluster.  (Measured shares, 4e-6 to .13, agree: 2M cells in boxes of
 //    100, 10 and 1, 200k and 20k in boxes of 1 and .1.)  Where that is most rays,
 //    none are marched.  With too few rays to fill the card the leftover's own
-//    walk comes on top, so there one such ray is too much: 200k cells in a unit
-//    box, 32^2 rays 1.3 ms in the engine, 2.2 marched with one ray left, 64^2 2.1
-//    and 3.2, 128^2 4.5 and 3.8.
+//    walk comes on top, so there one such ray is too much, unless the cloud is so
+//    large that the engine takes longer than both.  In the engine, and marched
+//    with rays left, ms: 50k cells, 4,096 rays 1.55 and 1.9; 200k, 1,024 rays 1.3
+//    and 2.2, 4,096 2.0 and 3.1, 16,384 4.5 and 3.8; 700k, 2,025 rays 1.9 and 2.7,
+//    4,096 4.2 and 3.0; 2M, 529 rays 2.7 and 3.5, 1,024 2.9 and 3.1, 2,025 3.9 and
+//    3.1; 8M, 2,025 rays 12 and 4.5.
 bool march_pays(const vt_cloud *c, int64_t n) {
   if (c->march_limit == 0 || help_events() <= 0) return false;
   const DevCloud &d = c->dc;
@@ -821,7 +824,9 @@ bool march_pays(const vt_cloud *c, int64_t n) {
   const double area = side[1] * side[2];
   if (!(area > 0.0)) return true;
   const double met = 13.0 * clearance * cells / area;
-  return met < 1.0 && (n > 32ll * num_cus(c->device) || met * (double)n < 0.5);
+  const double cus = num_cus(c->device), rays = (double)n;
+  const bool fills = rays > 32.0 * cus || rays * cells > 7e6 * cus;
+  return met < 1.0 && (fills || met * rays < 0.5);
 }
 
 // Whether the cloud's lists are worth building for a call of n rays: once the
