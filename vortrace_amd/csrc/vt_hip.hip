@@ -832,14 +832,16 @@ bool march_pays(const vt_cloud *c, int64_t n) {
 // Whether the cloud's lists are worth building for a call of n rays: once the
 // calls that ran without them, this one included, have cost the engine what the
 // lists cost to build.  So a cloud that is only queried or sliced, or projects a
-// few rays once, has none.  Lists take .35 ms at 5k cells, 2.4 to 4.3 at 200k and
-// 12 at 2M clustered ones; calls without them .6 ms (one ray, 20k cells), 2.8
-// (128^2, 100k), 41 (512^2, 2M).  Building a cloud and its first projection,
-// lists at upload -> here: 5k cells, 16^2 rays 1.68 -> 1.71 ms, 100k, 128^2
-// 15.96 -> 15.68; building alone 1.05 -> .71 and 14.5 -> 13.7.
+// few rays once, has none.  Lists take .35 ms at 5k cells, 2.4 to 4.3 at 200k, 12
+// at 2M and 29 at 8M clustered ones, and as much as .3 + 1e-6 N to allocate; calls
+// without them .6 ms (one ray, 20k cells), 2.8 (128^2, 100k), 6 (20k chords,
+// 200k), 41 (512^2, 2M).  Building a cloud and its first projection, lists at
+// upload -> here: 5k cells, 16^2 rays 1.68 -> 1.71 ms, 100k, 128^2 15.96 ->
+// 15.68; building alone 1.05 -> .71 and 14.5 -> 13.7.
 bool lists_pay(const vt_cloud *c, int64_t n) {
-  const double build_ms = 0.3 + 1e-5 * (double)c->n;
-  const double call_ms = 0.6 + 1.5e-6 * (double)n * 1.1 * std::cbrt((double)c->n);
+  const double cells = (double)c->n;
+  const double build_ms = std::min(0.4 + 2e-5 * cells, 8.0 + 5e-6 * cells);
+  const double call_ms = 0.6 + 3e-6 * (double)n * 1.1 * std::cbrt(cells);
   return c->engine_ms + call_ms >= build_ms;
 }
 
