@@ -282,17 +282,16 @@ int vt_cloud_set_march_limit(vt_cloud *cloud, size_t max_bytes);
 /* Launch parameters of the ray kernels (process-wide): lanes of a wave that
  * run their walk steps together, lanes that run their leaf steps together
  * (both 1..64), ray partitions (1, or 8: one per XCD), and help_events
- * (0..128).  With help_events > 0 rays are marched from cell to cell over the
- * cells' neighbour lists, and the lanes of a wave share the check of the
- * march -- 8 * help_events intervals at once (at most 256, or 512 in clouds of
- * more than some 10 million points), beyond which a ray is handed back -- and
- * the ray engine, which runs the rays the march leaves, lets lanes with no ray
- * left walk intervals of other lanes' rays, recording up to this many
- * boundaries of one before they hand it back (more in launches of few rays,
- * which share the buffers of all lanes).  0: every ray runs in the engine,
- * without help.  Results do not depend on them, only speed.  No reference
- * counterpart (the reference's OpenMP loop has schedule(dynamic,256) fixed,
- * src/projection.cpp:43); vortrace_amd.tuning.autotune picks them. */
+ * (0..128): in the ray engine, lanes with no ray left walk intervals of other
+ * lanes' rays, recording up to this many boundaries of one before they hand it
+ * back (more where a call's leftovers are few, or have the march's rows to record
+ * into); the same lanes share the march's check, 8 * help_events intervals at
+ * once (at most 256, or 512 in clouds of more than 11 million points), beyond
+ * which a ray is left to the engine.  0: no helping, and no march either.  (The
+ * engine alone, with helping: a march limit of 0.)  Results do not depend on
+ * them, only speed.  No reference counterpart (the reference's OpenMP loop has
+ * schedule(dynamic,256) fixed, src/projection.cpp:43);
+ * vortrace_amd.tuning.autotune picks them. */
 typedef struct {
   int walk_batch, leaf_batch, ray_parts, help_events;
 } vt_tuning;

@@ -297,6 +297,13 @@ __global__ __launch_bounds__(kBlock) void k_locate_far(DevCloud C, Scratch S, Ma
 // but a millionth of the exits; the rest, and every exit taken, are computed
 // again in FP64.  Keeping the places and their g'.d in FP64 through the
 // selects and the lanes' exchange took a third of the scan's instructions.
+//
+// A key (key_of) is off by the rounding of its numerator and of g'.d to float
+// (2^-24 of themselves each), the reciprocal's last place (2^-23) and the
+// product's rounding (2^-24; halving is exact): 5 2^-24 = 3.0e-7 of itself.  Two
+// keys compared may be 6.0e-7 of the larger apart from their FP64 values'
+// order, and kKeyTol leaves two fifths of itself above that.  A key that
+// underflows lies within any zone of the entry, where no exit is accepted.
 constexpr double kKeyTol = 1e-6;
 struct Best {
   float t1, t2, t3;
@@ -509,11 +516,13 @@ __device__ __forceinline__ float box_below2(const float (&lo)[3], const float (&
 //
 // Groups take rays from a queue of the batch's slots, one part per XCD.
 //
-// Bound by VALU issue (64 % of the cycles) and, with three waves per SIMD, by the
-// latency of the chain list -> generators -> exit -> next list.  2M clustered
-// cells, 512^2 rays (126 crossings each): 7.1 ms, of which the 1.1 % of
-// crossings that search take a quarter; 1M such cells, 1024^2 rays: 2 x 10.1 ms.
-// With FP64 keys, the image shifts computed at each use and all of the ray in
+// 2M clustered cells, 512^2 rays (126 crossings each): 7.1 ms, of which the 1.1 %
+// of crossings that search take a quarter; 1M such cells, 1024^2 rays: 2 x 10.1
+// ms.  Counters of the former: VALU issues in 57 % of the SIMDs' cycles (70 wave
+// instructions a crossing, 35 lanes active, 29 % of them FP64), the address units
+// are busy in 55 %, 68 % of the reads hit L1, and the 2.4 waves a SIMD holds wait
+// for half of their time: the chain list -> generators -> exit -> next list.  With
+// FP64 keys, the image shifts computed at each use and all of the ray in
 // registers it was 8.0 and 2 x 11.5 ms; the keys in scratch memory (see merge)
 // cost 1.2 ms, two waves per SIMD 1.4 ms, and four, which spill here, nothing
 // less.  A ray's own lane descending the tree alone took 65 ms (chains of up to

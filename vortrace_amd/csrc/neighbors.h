@@ -9,8 +9,9 @@
 // generator of the leaf ranks the collected ones by distance.  A leaf's
 // generators share one traversal and one set of candidates.  Bound by VALU
 // issue, the ranking a third of it: 2M clustered points 12.1 ms, 8M 29.0 (13.9
-// and 39.7 with ties ranked in the same pass).  64 entries: at 48, 2 % of the crossings of a clustered mesh
-// have more generators in reach than the list holds, at 64 1.2 %, at 96 0.9 %.
+// and 39.7 with ties ranked in the same pass).  64 entries: at 48, 2 % of the
+// crossings of a clustered mesh have more generators in reach than the list
+// holds, at 64 1.2 %, at 96 0.9 %.
 #pragma once
 #include "knn.h"
 #include "march.h"

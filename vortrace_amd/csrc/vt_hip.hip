@@ -110,7 +110,8 @@ __device__ __forceinline__ void run_io(const DevCloud &C, const Scratch &S, cons
 template <int MODE, int NF, bool PER, bool REC = false, bool HELP = false>
 __global__ __launch_bounds__(kBlock) __attribute__((amdgpu_waves_per_eu(2))) void k_project(
     DevCloud C, Scratch S, const double *start, const double *end, int64_t nrays,
-    const uint32_t *ray_list, uint32_t *defer, double *out, int nout, int64_t *counts, RecPool pool, ErrRec *err, Stats *stats) {
+    const uint32_t *ray_list, uint32_t *defer, double *out, int nout, int64_t *counts,
+    RecPool pool, ErrRec *err, Stats *stats) {
   if constexpr (MODE == VT_SUM && NF > 0) {
     run_io<REC, PER, false, HELP>(C, S, start, end, nrays, ray_list, defer, err, stats,
                                   SumIO<NF>{C.fields, out, nout, counts}, pool);
@@ -952,9 +953,6 @@ int march(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io
   return rc;
 }
 
-// A call's rays: marched, and those the march leaves run in the engine
-// (fast(timer, list, n) and slow(timer, n) as in two_pass); or all of them in
-// the engine.
 // Rays that start or end farther than `edge` outside the generators' box.
 __global__ void k_leaving(DevCloud C, const double *s, const double *e, int64_t n, double edge,
                           Stats *stats) {
@@ -988,6 +986,9 @@ bool engine_sooner(vt_cloud *c, const double *s, const double *e, int64_t n, hip
   return out > 0;
 }
 
+// A call's rays: marched, and those the march leaves run in the engine
+// (fast(timer, list, n) and slow(timer, n) as in two_pass); or all of them in
+// the engine.
 template <class IO, class Fast, class Slow>
 int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const IO &io,
                hipStream_t st, Fast &&fast, Slow &&slow, bool projects = false) {
@@ -1439,8 +1440,8 @@ int project_noalloc(vt_cloud *c, const double *d_s, const double *d_e, int64_t n
   };
   {
     const int grid = prepare(kfast, n, true);
-    kfast<<<grid, kBlock, 0, st>>>(c->dc, s, d_s, d_e, n, nullptr, defer, out, nout, nullptr, RecPool{},
-                                   c->d_err, c->d_stats);
+    kfast<<<grid, kBlock, 0, st>>>(c->dc, s, d_s, d_e, n, nullptr, defer, out, nout, nullptr,
+                                   RecPool{}, c->d_err, c->d_stats);
     HIP_OK(hipGetLastError());
     const int rc = finish_call(c, st, nullptr, nullptr);
     if (rc) return rc;

@@ -5,12 +5,13 @@ and groups leaf steps and walk steps: a wave runs its leaf steps once
 ``leaf_batch`` of its lanes are at a leaf, and its walk steps once
 ``walk_batch`` lanes wait for one.  Rays are taken from ``ray_parts``
 partitions (8: one per XCD, for L2 locality; or 1).  With ``help_events`` > 0
-rays are marched over the cells' neighbour lists (march.hip), the lanes of a
-wave share the march's check (8 * ``help_events`` intervals at once, at most
-256), and the engine runs what the march leaves, its idle lanes walking
-intervals of busy lanes' rays (up to ``help_events`` boundaries each, more in
-launches of few rays); 0 runs every ray in the engine, without help.  Results never depend on
-these values, only speed.  The kd-tree's leaf size stays the reference's 10
+its idle lanes walk intervals of busy lanes' rays, up to that many boundaries
+each (more for a march's leftovers), and rays are marched over the cells'
+neighbour lists first (march.hip) where that pays, a wave's lanes sharing the
+march's check (8 * ``help_events`` intervals at once, at most 256); 0 runs every
+ray in the engine, without help, and a march limit of 0
+(``PointCloud.set_march_limit``) runs them there with help.  Results never depend
+on these values, only speed.  The kd-tree's leaf size stays the reference's 10
 (src/pointcloud.cpp:204): the order of equidistant neighbours, and with it the
 crossing sequences, depends on it.
 """
