@@ -68,6 +68,18 @@ __device__ __forceinline__ uint32_t group_swap(uint32_t v) {
   constexpr int ctrl = STEP == 0 ? 0xB1 : (STEP == 1 ? 0x4E : (STEP == 2 ? 0x141 : 0x140));
   return (uint32_t)__builtin_amdgcn_update_dpp(0, (int)v, ctrl, 0xF, 0xF, true);
 }
+// The value of a group's first lane.
+template <int G>
+__device__ __forceinline__ uint32_t group_first(uint32_t v) {
+  static_assert(G == 4 || G == 8 || G == 16, "groups are quads, half rows or rows");
+  const int i = (int)v;
+  if constexpr (G == 4) return (uint32_t)__builtin_amdgcn_update_dpp(i, i, 0x00, 0xF, 0xF, true);
+  // Lane 0 of every row of 16, and for the second half of a row its lane 8.
+  const int row = __builtin_amdgcn_update_dpp(i, i, 0x150, 0xF, G == 8 ? 0x3 : 0xF, false);
+  if constexpr (G == 16) return (uint32_t)row;
+  return (uint32_t)__builtin_amdgcn_update_dpp(row, i, 0x158, 0xF, 0xC, false);
+}
+
 // The nearest generator so far.
 struct Near {
   double d2 = INFINITY;
@@ -355,13 +367,16 @@ struct Best {
     o.n2 = group_swap<STEP>(n2);
     merge(o);
   }
-  // The candidates of a group's lanes, in every lane.
+  // The candidates of a group's lanes, alike in every lane: of equal keys, each
+  // lane of a pair keeps its own in front, so the names are the first lane's.
   template <int G>
   __device__ __forceinline__ void reduce() {
-    if constexpr (G > 1) swap_in<0>();
-    if constexpr (G > 2) swap_in<1>();
+    swap_in<0>();
+    swap_in<1>();
     if constexpr (G > 4) swap_in<2>();
     if constexpr (G > 8) swap_in<3>();
+    n1 = group_first<G>(n1);
+    n2 = group_first<G>(n2);
   }
 };
 
