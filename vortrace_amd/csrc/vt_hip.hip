@@ -321,6 +321,7 @@ T *dev_alloc(size_t count) {
     (void)hipGetLastError();
     e = hipMalloc(&p, count * sizeof(T));
   }
+  if (e != hipSuccess) (void)hipGetLastError();  // (not the next launch's error)
   HIP_OK(e);
   return static_cast<T *>(p);
 }
@@ -997,12 +998,12 @@ int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const I
   int64_t left = n;
   bool marched = false;
   RowLease rows(st);
-  // (The kernels that count and list segments are slower than the march for any
-  // number of rays.)
   const bool wants = march_pays(c, n);
   if (wants && !c->lists.ready() && lists_pay(c, n)) build_lists(c, st);
   {
     const ListLease lists(c->lists, wants);
+    // (engine_sooner was measured for projections; the kernels that count and list
+    // segments are slower than the march for any number of rays that leave.)
     if (lists && !(projects && engine_sooner(c, s, e, n, st))) {
       // (The march's own searches run on the engine's lanes.)
       ensure_scratch(c, (size_t)march_locate_grid(num_cus(c->device)) * kBlock);
@@ -1030,7 +1031,7 @@ int march_then(vt_cloud *c, const double *s, const double *e, int64_t n, const I
       }
     }
   }
-  // (The rows are given back on every way out, so the buffers in them are too.)
+  // (Gone before the rows they lie in, on every way out.)
   struct Gifts {
     vt_cloud *c;
     ~Gifts() {
