@@ -155,3 +155,56 @@ def test_lists_wait_for_rays_that_pay_for_them():
     for _ in range(40):
         assert torch.equal(p.project_tensor(cloud), first)
     assert free1 - torch.cuda.mem_get_info()[0] > 200 * n, "no lists after forty calls"
+
+
+def test_lists_dropped_while_other_clouds_project():
+    """One thread takes lists away as a failing allocation would, others project."""
+    work = []
+    for k, n in enumerate((4_000, 9_000)):
+        pc = _cloud(n, 110 + k)
+        s, e = _grid(60, 40)
+        work.append((pc, s, e, _engine(pc, s, e)))
+    torch.cuda.synchronize()
+    stop, bad = threading.Event(), []
+
+    def run(pc, s, e, want):
+        with torch.cuda.stream(torch.cuda.Stream()):
+            for _ in range(60):
+                if not torch.equal(pc.projection_tensor(s, e), want):
+                    bad.append(len(s))
+
+    def hog():
+        c = vt.PointCloud()
+        c.loadPoints(np.random.default_rng(0).random((500, 3)), np.ones(500),
+                     [0.0, 1.0] * 3, periodic=True)
+        c.buildTree()
+        q = torch.rand(64, 3, dtype=torch.float64, device="cuda")
+        first = c.query_tensor(q, 2)[0]
+        refused = 0
+        while not stop.is_set():
+            try:
+                c.set_ray_order(order)  # a copy of 4 GiB: the library frees what it can
+            except RuntimeError:
+                refused += 1
+            # The refusal is not the next call's.
+            if not torch.equal(c.query_tensor(q, 2)[0], first):
+                bad.append("query")
+        taken.append(refused)
+    taken = []
+    _say("filling the device's memory")
+    order = torch.zeros(1 << 30, dtype=torch.int32, device="cuda")
+    hog_mem = _hog(3 * GIB)
+    threads = [threading.Thread(target=run, args=w) for w in work]
+    taker = threading.Thread(target=hog)
+    _say("projecting")
+    taker.start()
+    for t in threads:
+        t.start()
+    for t in threads:
+        t.join()
+    stop.set()
+    taker.join()
+    del hog_mem, order
+    torch.cuda.empty_cache()
+    assert not bad
+    assert taken and taken[0] > 0

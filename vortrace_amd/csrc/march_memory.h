@@ -16,8 +16,8 @@
 
 namespace {
 
-// Device memory that is free, for requests of `want` bytes; unlimited for small
-// ones, which need not ask (asking took .3 ms of a small cloud's first call).
+// Device memory that is free, for requests of `want` bytes; small ones need not
+// ask.
 size_t free_for(size_t want) {
   size_t avail = 0, total = 0;
   if (want < ((size_t)256 << 20)) return SIZE_MAX / 2;
@@ -34,6 +34,8 @@ struct MarchLists {
   // Lists stay for their cloud's life, so they may take half of what is free.
   bool alloc(size_t want) {
     if (p && bytes >= want) return true;  // (from a build that failed half way)
+    if (p) (void)hipFree(p);
+    bytes = 0;
     if (want > free_for(want) / 2 || hipMalloc(&p, want) != hipSuccess) {
       (void)hipGetLastError();
       p = nullptr;
@@ -42,15 +44,18 @@ struct MarchLists {
     bytes = want;
     return true;
   }
-  // Frees them unless a call uses them (also a build that failed half way).
+  // Frees them unless a call uses them.  They count as used meanwhile, so that a
+  // call of their cloud neither takes nor builds them.  (What a build that failed
+  // half way left, its own cloud's calls alone free.)
   bool drop() {
-    int idle = kIdle;
-    if (!state.compare_exchange_strong(idle, kNone) && idle == kUsed) return false;
-    if (!p) return false;
-    (void)hipFree(p);
+    int was = kIdle;
+    if (!state.compare_exchange_strong(was, kUsed) && was == kUsed) return false;
+    const bool freed = p != nullptr;
+    if (p) (void)hipFree(p);
     p = nullptr;
     bytes = 0;
-    return true;
+    state.store(kNone);
+    return freed;
   }
 };
 
