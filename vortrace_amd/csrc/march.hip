@@ -533,9 +533,9 @@ __device__ __forceinline__ float box_below2(const float (&lo)[3], const float (&
 //
 // 2M clustered cells, 512^2 rays (126 crossings each): 7.1 ms, of which the 1.1 %
 // of crossings that search take a quarter; 1M such cells, 1024^2 rays: 2 x 10.1
-// ms.  Counters of the former: VALU issues in 57 % of the SIMDs' cycles (70 wave
+// ms.  Counters of the former: VALU issues in 58 % of the SIMDs' cycles (71 wave
 // instructions a crossing, 35 lanes active, 29 % of them FP64), the address units
-// are busy in 55 %, 68 % of the reads hit L1, and the 2.4 waves a SIMD holds wait
+// are busy in 56 %, 68 % of the reads hit L1, and the 2.5 waves a SIMD holds wait
 // for half of their time: the chain list -> generators -> exit -> next list.  With
 // FP64 keys, the image shifts computed at each use and all of the ray in
 // registers it was 8.0 and 2 x 11.5 ms; the keys in scratch memory (see merge)
