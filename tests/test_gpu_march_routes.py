@@ -145,3 +145,26 @@ def test_rows_of_more_than_640_cells():
     pc = vt.ProjectionCloud(pos, rho, boundbox=BB, periodic=True)
     marched, left = _routes(pc, *_axis(500_000, 3))
     assert marched == 500_000 and left < 500  # (some ten meet a near-tie)
+
+
+def test_autotune_times_marched_calls():
+    """A few rays through a large cloud: lists are built before anything is timed."""
+    pos, rho = synthetic.uniform_mesh(600_000, seed=67)
+    pc = vt.ProjectionCloud(pos, rho, boundbox=BB, periodic=True)
+    saved = vt.tuning.get_tuning()
+    marched = []
+    try:
+        project = pc.projection_tensor
+
+        def seen(*a, **kw):
+            out = project(*a, **kw)
+            marched.append((vt.tuning.get_tuning()["help_events"], _lib.last_march_stats().rays))
+            return out
+        pc.projection_tensor = seen
+        out = vt.tuning.autotune(pc, *_axis(64, 5), stride=1, walk_batches=(32,),
+                                 leaf_batches=(32,), ray_parts=(8,), help_events=(0, 128),
+                                 repeats=2, cache=False)
+    finally:
+        vt.tuning.set_tuning(**saved)
+    assert [r for r in marched[-4:]] == [(0, 0), (0, 0), (128, 64), (128, 64)]
+    assert len(out["results"]) == 2

@@ -67,7 +67,14 @@ def autotune(pc, pos_start, pos_end, *, reduction: str = "integrate", stride: in
     s = torch.as_tensor(pos_start, dtype=torch.float64).reshape(-1, 3)[::stride]
     e = torch.as_tensor(pos_end, dtype=torch.float64).reshape(-1, 3)[::stride]
     s, e = s.to(dev).contiguous(), e.to(dev).contiguous()
-    pc.projection_tensor(s, e, reduction=reduction)  # warm-up
+    # Warm-up, until the cloud's neighbour lists are built (or are not going to be:
+    # their cost is at most this): the later calls are what is timed.
+    spent, built = 0.0, 8.0 + 5e-6 * pc._cloud.get_npart()
+    while spent <= built:
+        pc.projection_tensor(s, e, reduction=reduction)
+        spent += max(_lib.last_call_stats().kernel_ms, 0.1)
+        if _lib.last_march_stats().rays:
+            break
     results = []
     for wb, lb, rp, he in itertools.product(walk_batches, leaf_batches, ray_parts, help_events):
         set_tuning(wb, lb, rp, he)
