@@ -802,9 +802,9 @@ void launch(vt_cloud *c, K kernel, int64_t n, hipStream_t st, Timer &tm, A... ar
 //    every edge of a cell that is a strip of clearance / spacing, so a crossing
 //    meets one with a probability of some 13 clearance / spacing^2, and a ray
 //    through a box of N cells in 13 clearance N / area crossings, however the
-//    cells cluster.  (Measured shares, 4e-6 to .13, agree: 2M cells in boxes of
-//    100, 10 and 1, 200k and 20k in boxes of 1 and .1.)  Where that is most rays,
-//    none are marched.  With too few rays to fill the card the leftover's own
+//    cells cluster.  (Measured shares of rays left, 4e-6 to .13, agree within a
+//    factor of two: 2M cells in boxes of 100, 10 and 1, 200k and 20k in boxes of 1
+//    and .1.)  Where that is most rays, none are marched.  With too few rays to fill the card the leftover's own
 //    walk comes on top, so there one such ray is too much, unless the cloud is so
 //    large that the engine takes longer than both.  In the engine, and marched
 //    with rays left, ms: 50k cells, 4,096 rays 1.55 and 1.9; 200k, 1,024 rays 1.3
@@ -835,9 +835,9 @@ bool march_pays(const vt_cloud *c, int64_t n) {
 // calls that ran without them, this one included, have cost the engine what the
 // lists cost to build.  So a cloud that is only queried or sliced, or projects a
 // few rays once, has none.  Lists take .35 ms at 5k cells, 2.4 to 4.3 at 200k, 12
-// at 2M and 29 at 8M clustered ones, and as much as .3 + 1e-6 N to allocate; calls
-// without them .6 ms (one ray, 20k cells), 2.8 (128^2, 100k), 6 (20k chords,
-// 200k), 41 (512^2, 2M).  Building a cloud and its first projection, lists at
+// at 2M and 29 at 8M clustered ones, and are allocated and joined by the boxes;
+// calls without them .6 ms (one ray, 20k cells), 2.8 (128^2, 100k), 41 (512^2,
+// 2M).  Building a cloud and its first projection, lists at
 // upload -> here: 5k cells, 16^2 rays 1.68 -> 1.71 ms, 100k, 128^2 15.96 ->
 // 15.68; building alone 1.05 -> .71 and 14.5 -> 13.7.
 bool lists_pay(const vt_cloud *c, int64_t n) {
